@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 #include "cwen_gpu.h"
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
@@ -167,6 +168,14 @@ __device__ __forceinline__ void raise_flag(int *flag) {
   if (flag) __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A product as f32, so that a conversion after it rounds a second time: the
+// compiler otherwise may fold the two into one mixed-precision operation
+// (v_fma_mixlo_f16), in one kernel and not in another.
+__device__ __forceinline__ float f32_of(float x) {
+  asm("" : "+v"(x));
+  return x;
+}
+
 // Row-tile partials of a column's sum of squares: at most 128 per column.
 constexpr int CWEN_MAX_PARTS = 128;
 
@@ -249,6 +258,32 @@ int gemv_launch(cwen_ctx *ctx, const cwen_weight *w, int nsides, int side0, int 
 int act_to_f16(const float *x, int xs, _Float16 *xh, int K, int B, hipStream_t st);
 int argmax_walk_launch(const float *lg, long ls, int V, int B, const ArgmaxOut &a, hipStream_t st);
 
+// ------------------------------------------------------------ wide.hip
+// Products for N positions at once (a prompt's prefill): the bits that
+// gemv_launch gives each position in a block.
+constexpr int WIDE_MAX = 1024;   // positions of one pass at most
+struct WideOut {
+  float *y;          // STORE: f32 result [c*ys + row]
+  int ys;
+  int accumulate;    // y += result
+  _Float16 *yh;      // SWIGLU: silu(A)*B; STORE (nullable): y * nwh[row]; [c*M + row]
+  const float *nwh;
+  float *ssq;        // STORE, nullable: sums of squares of y per 64 rows [c][CWEN_MAX_PARTS]
+  int *rflag;        // set to 1 when an f16 value written is not finite
+};
+// Whether wide_gemm takes the weight (finish: as an accumulating STORE, whose
+// rows must not be partly whole, partly split over K).
+bool wide_takes(const cwen_weight *w, int nsides, bool finish);
+// Floats of `part` that wide_gemm needs for N positions of w; finish: an
+// accumulating STORE.
+size_t wide_partial_floats(const cwen_weight *w, int nsides, bool finish, int N);
+// The per-position scale of a normalised operand (GemvPost) for N positions;
+// psc holds N floats rounded up to a multiple of 64.
+int wide_scale(const float *ssq, int npart, int K, float eps, int N, float *psc, hipStream_t st);
+// epi STORE or SWIGLU; psc nullable.
+int wide_gemm(const cwen_ctx *ctx, const cwen_weight *w, int epi, const _Float16 *xh, int N, const float *psc,
+              const WideOut &o, float *part, hipStream_t st);
+
 // ------------------------------------------------------------ gdn.hip
 int gdn_block_launch(const cwen_gdn *g, const float *qkv, int qs, const float *z, int zs,
                      const float *decay, const float *beta, int gs, const float *kw, const float *wn,
@@ -259,6 +294,14 @@ int gdn_block_launch(const cwen_gdn *g, const float *qkv, int qs, const float *z
 // rows < g->C): the GEMV then does what gdn_conv_kernel would, and
 // gdn_block_launch is called with conv_done.
 void gdn_conv_out(const cwen_gdn *g, const float *kw, GemvOut &o);
+// N positions (a whole number of 16-position blocks) of a prefill, all
+// accepted: `lin` holds the in-projection's rows [N][ls] (qkv, then z at
+// column zo and the raw gates at ao and bo); its qkv columns are overwritten.
+// xc [N][C] and gates [N][2][nvh] are scratch.  The layer must have no pending replay; the
+// state advances in place and the history moves to slot cur + 1.
+int gdn_wide_launch(const cwen_gdn *g, float *lin, int ls, int zo, int ao, int bo, const float *kw, const float *wn,
+                    const float *A, const float *dt, float *xc, float *gates, _Float16 *outh, int N, int *rflag,
+                    hipStream_t st);
 // The state after replaying L positions of pending buffer buf from base slot
 // X into S_out (device, [nvh][dk][dk]).
 int gdn_peek_launch(const cwen_gdn *g, int L, int buf, float *S_out, hipStream_t st);
@@ -284,6 +327,13 @@ int attention_launch(const float *qfull, int qfs, const float *kx, const float *
                      const float *kn, float *qbuf, float *K, float *V, const int *last, int B, int NH, int NKV,
                      int npairs, int nrot, float theta, float eps, float *part, int max_ctx, _Float16 *yh,
                      hipStream_t st, int *rflag = nullptr, int last_hint = -1);
+// The same for N positions (a whole number of 16-position blocks): qbuf
+// [N][NH][256], yh [N][NH*256]; `part` as for B = 16; last_host: the host's
+// copy of *last.
+int attention_wide_launch(const float *qfull, int qfs, const float *kx, const float *vx, int kvs, const float *qn,
+                          const float *kn, float *qbuf, float *K, float *V, const int *last, int last_host, int N, int NH,
+                          int NKV, int npairs, int nrot, float theta, float eps, float *part, int max_ctx, _Float16 *yh,
+                          hipStream_t st, int *rflag);
 // Whether a block whose last position is last_pos takes the wide chunk grid
 // (attention_launch's last_hint; -1 = not known, narrow).  Only the launch
 // shape depends on it, never the result.

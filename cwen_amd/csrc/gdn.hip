@@ -300,6 +300,195 @@ __global__ __launch_bounds__(64 * RW) void gdn_rec_kernel(GdnParams p) {
   }
 }
 
+// ---- many accepted positions (a prefill's prompt).  The same arithmetic per
+// position and column as the kernels above, so the state and outputs are the
+// bits that the blocks of 16 would give; what differs is the division of
+// labour.  In a block, 48 workgroups (one per head) also normalise, gate and
+// norm; here the per-position work runs over all positions first, and the
+// recurrence, the only serial part, takes 4 workgroups per head.
+
+struct GdnWide {
+  const float *S_in; float *S_out;    // [nvh][DK][DK] (may be the same)
+  const float *H_in; float *H_out;    // history [C][3] before / after
+  float *lin; int ls;                 // in-projection rows [N][ls]
+  int zo, ao, bo;                     // z, alpha, beta columns of a row
+  const float *kw, *wn, *A, *dt;
+  float *xc;                          // [N][C]: post-conv, q and k l2-normalised
+  float *gates;                       // [N][2][nvh]: g, beta
+  _Float16 *outh;                     // [N][nvh*DK]
+  int *rflag;
+  int nkh, nvh, C, N;
+};
+
+// Conv + SiLU (+ l2 norm of q and k): a wave takes one 128-channel head of 4
+// consecutive positions, two channels per lane.  The last "head" (blockIdx.x
+// past the channels) does the positions' gates.
+__global__ __launch_bounds__(256) void gdn_wide_conv_kernel(GdnWide p) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int h = blockIdx.x, b0 = (blockIdx.y * 4 + wave) * 4;
+  if (b0 >= p.N) return;
+  if (h * DK >= p.C) {
+    for (int e = lane; e < 4 * p.nvh; e += 64) {
+      const int b = b0 + e / p.nvh, hv = e % p.nvh;
+      if (b >= p.N) break;
+      float dec = p.lin[(size_t)b * p.ls + p.ao + hv], bt = p.lin[(size_t)b * p.ls + p.bo + hv];
+      const float x = dec + p.dt[hv];
+      dec = p.A[hv] * (x > 20.f ? x : logf(1.f + expf(x)));
+      bt = 1.f / (1.f + expf(-bt));
+      p.gates[((size_t)b * 2 + 0) * p.nvh + hv] = expf(dec);
+      p.gates[((size_t)b * 2 + 1) * p.nvh + hv] = bt;
+    }
+    return;
+  }
+  float in[7][2];
+  float4 w[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int c = h * DK + lane + 64 * k;
+    w[k] = *(const float4 *)(p.kw + (size_t)c * 4);
+#pragma unroll
+    for (int j = 0; j < 7; ++j) {
+      const int t = b0 - 3 + j;
+      in[j][k] = t >= 0 ? p.lin[(size_t)min(t, p.N - 1) * p.ls + c] : p.H_in[(size_t)c * 3 + t + 3];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int b = b0 + e;
+    if (b >= p.N) break;
+    float y[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const float x = __fadd_rn(__fadd_rn(__fadd_rn(__fmul_rn(in[e][k], w[k].x), __fmul_rn(in[e + 1][k], w[k].y)),
+                                          __fmul_rn(in[e + 2][k], w[k].z)),
+                                __fmul_rn(in[e + 3][k], w[k].w));
+      y[k] = silu_ref(x);
+    }
+    if (h < 2 * p.nkh) {
+      const float r = 1.f / sqrtf(sum64(y[0] * y[0]) + sum64(y[1] * y[1]) + 1e-6f);
+      y[0] *= r;
+      y[1] *= r;
+    }
+    float *o = p.xc + (size_t)b * p.C + h * DK + lane;
+    o[0] = y[0];
+    o[64] = y[1];
+    if (b == p.N - 1) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        float *hs = p.H_out + (size_t)(h * DK + lane + 64 * k) * 3;
+        hs[0] = in[e + 1][k];
+        hs[1] = in[e + 2][k];
+        hs[2] = in[e + 3][k];
+      }
+    }
+  }
+}
+
+// The recurrence over N positions: workgroup (slice, head) = 4 waves, wave w
+// columns slice*32 + 8w .. +7 of the head; a lane owns 8 rows x 2 columns of S
+// in registers (rows as in gdn_rec_kernel, so a column's sums have its order).
+// Bound by the chain of one position (decay, 8 FMAs, 4 DPP adds, update);
+// 192 workgroups at 48 heads put one wave on each SIMD of 192 CUs.  The next
+// 16 positions' inputs are requested while 16 are computed; outputs meet in
+// LDS and leave 32 columns at a time, over the row's qkv columns.
+constexpr int WCOLS = 32;            // columns of a head per workgroup
+__global__ __launch_bounds__(256) void gdn_wide_rec_kernel(GdnWide p) {
+  __shared__ __align__(16) float qk[2][MAXB][2 * DK];
+  __shared__ __align__(16) float vs[2][MAXB][WCOLS];
+  __shared__ __align__(16) float ob[MAXB][WCOLS];
+  __shared__ float s_gb[2][2][MAXB];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int slice = blockIdx.x, hv = blockIdx.y, hk = hv % p.nkh;
+  const int rg = lane & 15, cg = lane >> 4;
+  const int i0 = rg * 8, jl = wave * 8 + cg * 2, j0 = slice * WCOLS + jl;
+  float2 s[8];
+  {
+    const float *Sh = p.S_in + (size_t)hv * DK * DK;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) s[r] = *(const float2 *)(Sh + (size_t)(i0 + r) * DK + j0);
+  }
+  // Staging of 16 positions: thread t loads 4 floats of q|k of positions
+  // (t >> 6) + 4 i, 2 floats of v of position t >> 4, and one gate (t < 32).
+  float4 rq[4];
+  float2 rv;
+  float rgt = 0.f;
+  auto request = [&](int b0) {
+    const int e = (tid & 63) * 4;
+    const int off = e < DK ? hk * DK + e : (p.nkh + hk) * DK + e - DK;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rq[i] = *(const float4 *)(p.xc + (size_t)(b0 + (tid >> 6) + 4 * i) * p.C + off);
+    rv = *(const float2 *)(p.xc + (size_t)(b0 + (tid >> 4)) * p.C + 2 * p.nkh * DK + hv * DK + slice * WCOLS + (tid & 15) * 2);
+    if (tid < 32) rgt = p.gates[((size_t)(b0 + (tid & 15)) * 2 + (tid >> 4)) * p.nvh + hv];
+  };
+  auto land = [&](int bf) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *(float4 *)&qk[bf][(tid >> 6) + 4 * i][(tid & 63) * 4] = rq[i];
+    *(float2 *)&vs[bf][tid >> 4][(tid & 15) * 2] = rv;
+    if (tid < 32) s_gb[bf][tid >> 4][tid & 15] = rgt;
+  };
+  request(0);
+  land(0);
+  __syncthreads();
+  const float scale = 1.f / sqrtf((float)DK);
+  for (int b0 = 0, bf = 0; b0 < p.N; b0 += MAXB, bf ^= 1) {
+    const bool more = b0 + MAXB < p.N;
+    if (more) request(b0 + MAXB);
+#pragma unroll 2
+    for (int b = 0; b < MAXB; ++b) {
+      const float g = s_gb[bf][0][b], beta = s_gb[bf][1][b];
+      const float4 qa = *(const float4 *)&qk[bf][b][i0], qb = *(const float4 *)&qk[bf][b][i0 + 4];
+      const float4 ka = *(const float4 *)&qk[bf][b][DK + i0], kb = *(const float4 *)&qk[bf][b][DK + i0 + 4];
+      const float kr[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
+      const float qr[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+      const float2 v2 = *(const float2 *)&vs[bf][b][jl];
+      float2 sk = {0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        s[r].x *= g; s[r].y *= g;
+        sk.x = fmaf(s[r].x, kr[r], sk.x); sk.y = fmaf(s[r].y, kr[r], sk.y);
+      }
+      sk = (float2){sum16(sk.x), sum16(sk.y)};
+      const float2 dl = {beta * (v2.x - sk.x), beta * (v2.y - sk.y)};
+      float2 o = {0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        s[r].x = fmaf(kr[r], dl.x, s[r].x); s[r].y = fmaf(kr[r], dl.y, s[r].y);
+        o.x = fmaf(s[r].x, qr[r], o.x); o.y = fmaf(s[r].y, qr[r], o.y);
+      }
+      o = (float2){sum16(o.x) * scale, sum16(o.y) * scale};
+      if (rg == 0) *(float2 *)&ob[b][jl] = o;
+    }
+    __syncthreads();                 // ob complete; the block's inputs read
+    {
+      const float2 o = *(const float2 *)&ob[tid >> 4][(tid & 15) * 2];
+      *(float2 *)(p.lin + (size_t)(b0 + (tid >> 4)) * p.ls + hv * DK + slice * WCOLS + (tid & 15) * 2) = o;
+    }
+    if (more) land(bf ^ 1);
+    __syncthreads();
+  }
+  float *So = p.S_out + (size_t)hv * DK * DK;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) *(float2 *)(So + (size_t)(i0 + r) * DK + j0) = s[r];
+}
+
+// Gated RMSNorm of the recurrence's outputs: one wave per (position, head).
+__global__ __launch_bounds__(256) void gdn_wide_norm_kernel(GdnWide p) {
+  const int lane = threadIdx.x & 63, hv = blockIdx.x, b = blockIdx.y * 4 + (threadIdx.x >> 6);
+  if (b >= p.N) return;
+  const float2 wn2 = *(const float2 *)(p.wn + 2 * lane);
+  const float2 o = *(const float2 *)(p.lin + (size_t)b * p.ls + hv * DK + 2 * lane);
+  const float z0 = p.lin[(size_t)b * p.ls + p.zo + hv * DK + 2 * lane];
+  const float z1 = p.lin[(size_t)b * p.ls + p.zo + hv * DK + 2 * lane + 1];
+  const float ss = sum64(o.x * o.x + o.y * o.y);
+  const float sc = 1.f / sqrtf(ss / DK + 1e-6f);
+  float2 r;
+  r.x = wn2.x * o.x * sc * silu_ref(z0);
+  r.y = wn2.y * o.y * sc * silu_ref(z1);
+  const half2_t h = {(_Float16)f32_of(r.x), (_Float16)f32_of(r.y)};
+  *(half2_t *)(p.outh + (size_t)b * p.nvh * DK + hv * DK + 2 * lane) = h;
+  if (f16_bad(h[0]) || f16_bad(h[1])) raise_flag(p.rflag);
+}
+
 }  // namespace
 
 static void fill_params(GdnParams &p, const cwen_gdn *g) {
@@ -345,6 +534,27 @@ int gdn_block_launch(const cwen_gdn *g, const float *qkv, int qs, const float *z
   if (!conv_done)
     hipLaunchKernelGGL(gdn_conv_kernel, dim3((unsigned)((g->C + 255) / 256), (unsigned)B), dim3(256), 0, st, p);
   hipLaunchKernelGGL(gdn_rec_kernel, dim3((unsigned)g->nvh), dim3(64 * RW), 0, st, p);
+  CWEN_HIP_TRY(hipGetLastError());
+  return CWEN_OK;
+}
+
+int gdn_wide_launch(const cwen_gdn *g, float *lin, int ls, int zo, int ao, int bo, const float *kw, const float *wn,
+                    const float *A, const float *dt, float *xc, float *gates, _Float16 *outh, int N, int *rflag,
+                    hipStream_t st) {
+  if (g->L || g->last_B || N < MAXB || N % MAXB || (ls & 1) || (zo & 1)) return CWEN_EINVAL;
+  const size_t hf = (size_t)g->C * 3;
+  float *S = g->S + (size_t)g->X * g->nvh * DK * DK;
+  GdnWide p;
+  p.S_in = S; p.S_out = S;
+  p.H_in = g->H + (size_t)g->cur * hf;
+  p.H_out = g->H + (size_t)((g->cur + 1) % g->nslot) * hf;
+  p.lin = lin; p.ls = ls; p.zo = zo; p.ao = ao; p.bo = bo;
+  p.kw = kw; p.wn = wn; p.A = A; p.dt = dt;
+  p.xc = xc; p.gates = gates; p.outh = outh; p.rflag = rflag;
+  p.nkh = g->nkh; p.nvh = g->nvh; p.C = g->C; p.N = N;
+  hipLaunchKernelGGL(gdn_wide_conv_kernel, dim3((unsigned)(g->C / DK + 1), (unsigned)((N + 15) / 16)), dim3(256), 0, st, p);
+  hipLaunchKernelGGL(gdn_wide_rec_kernel, dim3(DK / WCOLS, (unsigned)g->nvh), dim3(256), 0, st, p);
+  hipLaunchKernelGGL(gdn_wide_norm_kernel, dim3((unsigned)g->nvh, (unsigned)((N + 3) / 4)), dim3(256), 0, st, p);
   CWEN_HIP_TRY(hipGetLastError());
   return CWEN_OK;
 }

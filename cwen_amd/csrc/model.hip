@@ -9,6 +9,8 @@
 // Every kernel computes each position (block column) with the same
 // instructions whatever B is, so a block of B positions produces exactly the
 // values of B single-position passes.
+#include <algorithm>
+
 #include "cwen_internal.h"
 
 namespace {
@@ -118,7 +120,8 @@ struct AttnParams {
   const float *qn, *kn;
   float *q;            // [B][NH][HD] normed + roped queries
   float *K, *V;        // this layer's cache [ctx][NKV][HD]
-  const int *last;     // device: last filled cache slot before the block
+  const int *last;     // device: last filled cache slot before the block (the launch's positions
+  int off;             // start at *last + 1 + off)
   int max_ctx;         // cache slots; positions at or past it are not touched
   int B, NH, NKV, npairs, nrot;
   float theta, eps;
@@ -135,7 +138,7 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(AttnParams p) {
   __shared__ float red[4];
   __shared__ float v[HD];
   const int b = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
-  const int pos = *p.last + 1 + b;
+  const int pos = *p.last + 1 + p.off + b;
   if (pos < 0 || pos >= p.max_ctx) return;   // workgroup-uniform
   const bool isq = h < p.NH;
   const int hk = h - p.NH;
@@ -231,7 +234,7 @@ __global__ __launch_bounds__(64 * NW) void attn_chunk_kernel(AttnParams p) {
   // The position is read after the queries are requested (a scalar load
   // issued first would hold their address computation behind it).
   __builtin_amdgcn_sched_barrier(0);
-  const int pbase = *p.last + 1;
+  const int pbase = *p.last + 1 + p.off;
   const int tlast = min(pbase + p.B - 1, p.max_ctx - 1);  // last position of the block
   if ((int)blockIdx.x * TC > tlast) return;
   // Lands chunk c's K and V rows in LDS buffer `bf` (rows past the block's
@@ -388,7 +391,7 @@ __global__ __launch_bounds__(HD * MGR) void attn_merge_kernel(AttnParams p) {
   const int hkv = h / kvm, m = h % kvm;
   const int nq = p.B * kvm;
   const int qi = b * kvm + m;
-  const int pos = *p.last + 1 + b;
+  const int pos = *p.last + 1 + p.off + b;
   if (pos < 0 || pos >= p.max_ctx) return;
   const int nc = pos / TC + 1;
   __shared__ float red[HD * MGR / 64], s_w[HD * MGR], s_l[HD * MGR], s_lo[2][MGR][HD];
@@ -490,15 +493,14 @@ constexpr int ATTN_NARROW_CHUNKS = 192, ATTN_NARROW_WGS = 64, ATTN_WIDE_WGS = 12
 
 bool attention_wide(int last_pos) { return last_pos >= 0 && last_pos / TC + 1 > ATTN_NARROW_CHUNKS; }
 
-int attention_launch(const float *qfull, int qfs, const float *kx, const float *vx, int kvs, const float *qn,
-                     const float *kn, float *qbuf, float *K, float *V, const int *last, int B, int NH, int NKV,
-                     int npairs, int nrot, float theta, float eps, float *part, int max_ctx, _Float16 *yh,
-                     hipStream_t st, int *rflag, int last_hint) {
-  AttnParams p;
+namespace {
+void attn_params(AttnParams &p, const float *qfull, int qfs, const float *kx, const float *vx, int kvs, const float *qn,
+                 const float *kn, float *qbuf, float *K, float *V, const int *last, int B, int NH, int NKV, int npairs,
+                 int nrot, float theta, float eps, float *part, int max_ctx, _Float16 *yh, int *rflag) {
   p.qfull = qfull; p.qfs = qfs; p.kx = kx; p.vx = vx; p.kvs = kvs;
   p.qn = qn; p.kn = kn;
   p.q = qbuf; p.K = K; p.V = V;
-  p.last = last; p.max_ctx = max_ctx; p.B = B; p.NH = NH; p.NKV = NKV; p.npairs = npairs; p.nrot = nrot;
+  p.last = last; p.off = 0; p.max_ctx = max_ctx; p.B = B; p.NH = NH; p.NKV = NKV; p.npairs = npairs; p.nrot = nrot;
   p.theta = theta; p.eps = eps;
   p.nchunk = (max_ctx + TC - 1) / TC;
   const int nq = B * (NH / NKV);
@@ -507,6 +509,17 @@ int attention_launch(const float *qfull, int qfs, const float *kx, const float *
   p.pl = p.pm + (size_t)NKV * p.nchunk * nq;
   p.yh = yh;
   p.rflag = rflag;
+}
+}  // namespace
+
+int attention_launch(const float *qfull, int qfs, const float *kx, const float *vx, int kvs, const float *qn,
+                     const float *kn, float *qbuf, float *K, float *V, const int *last, int B, int NH, int NKV,
+                     int npairs, int nrot, float theta, float eps, float *part, int max_ctx, _Float16 *yh,
+                     hipStream_t st, int *rflag, int last_hint) {
+  AttnParams p;
+  attn_params(p, qfull, qfs, kx, vx, kvs, qn, kn, qbuf, K, V, last, B, NH, NKV, npairs, nrot, theta, eps, part, max_ctx,
+              yh, rflag);
+  const int nq = B * (NH / NKV);
   // Every check before the first launch: a block never stops half-way.
   const bool wide = attention_wide(last_hint);
   const int wgs = wide ? ATTN_WIDE_WGS : ATTN_NARROW_WGS;
@@ -521,6 +534,37 @@ int attention_launch(const float *qfull, int qfs, const float *kx, const float *
   hipLaunchKernelGGL(attn_prep_kernel, dim3((unsigned)B, (unsigned)(NH + NKV)), dim3(HD), 0, st, p);
   hipLaunchKernelGGL(attn_chunk_kernel<NW_MAX>, dim3((unsigned)nwg, (unsigned)NKV), dim3(64 * NW_MAX), lds, st, p);
   hipLaunchKernelGGL(attn_merge_kernel, dim3((unsigned)B, (unsigned)NH), dim3(HD * MGR), 0, st, p);
+  CWEN_HIP_TRY(hipGetLastError());
+  return CWEN_OK;
+}
+
+int attention_wide_launch(const float *qfull, int qfs, const float *kx, const float *vx, int kvs, const float *qn,
+                          const float *kn, float *qbuf, float *K, float *V, const int *last, int last_host, int N, int NH,
+                          int NKV, int npairs, int nrot, float theta, float eps, float *part, int max_ctx, _Float16 *yh,
+                          hipStream_t st, int *rflag) {
+  constexpr int B = CWEN_BMAX;
+  if (N < B || N % B || NH % NKV) return CWEN_EINVAL;
+  const int MT = (B * (NH / NKV) + 15) / 16;
+  if (MT > NW_MAX) return CWEN_EINVAL;
+  int rc;
+  if ((rc = attention_init())) return rc;
+  AttnParams p;
+  attn_params(p, qfull, qfs, kx, vx, kvs, qn, kn, qbuf, K, V, last, B, NH, NKV, npairs, nrot, theta, eps, part, max_ctx,
+              yh, rflag);
+  hipLaunchKernelGGL(attn_prep_kernel, dim3((unsigned)N, (unsigned)(NH + NKV)), dim3(HD), 0, st, p);
+  for (int j = 0; j < N; j += B) {
+    p.off = j;
+    p.q = qbuf + (size_t)j * NH * HD;
+    p.qfull = qfull + (size_t)j * qfs;
+    p.yh = yh + (size_t)j * NH * HD;
+    const bool wide = attention_wide(last_host + j + B);
+    const int wgs = wide ? ATTN_WIDE_WGS : ATTN_NARROW_WGS;
+    p.nbuf = wide ? 1 : 2;
+    const size_t lds = ((size_t)MT * 16 * PROW + p.nbuf * KV_FLOATS) * sizeof(float);
+    hipLaunchKernelGGL(attn_chunk_kernel<NW_MAX>, dim3((unsigned)std::min(p.nchunk, wgs), (unsigned)NKV),
+                       dim3(64 * NW_MAX), lds, st, p);
+    hipLaunchKernelGGL(attn_merge_kernel, dim3((unsigned)B, (unsigned)NH), dim3(HD * MGR), 0, st, p);
+  }
   CWEN_HIP_TRY(hipGetLastError());
   return CWEN_OK;
 }

@@ -11,6 +11,7 @@
 #include <string.h>
 #include <unistd.h>
 
+#include <algorithm>
 #include <new>
 
 #include "cwen_internal.h"
@@ -76,6 +77,14 @@ struct cwen_model {
   _Float16 *hh = nullptr;        // FFN hidden f16 [BMAX][I]
   float *logits = nullptr;       // [BMAX][V]
   int *hres = nullptr;           // pinned host copy of res
+  // Workspace of cwen_model_prefill for `wn` positions at a time (0: not
+  // allocated), the block scratch above at that length.
+  int wn = 0;
+  int *wtoks = nullptr, *hwtok = nullptr;              // device / pinned host tokens
+  float *wX = nullptr, *wssq = nullptr, *wpsc = nullptr;
+  float *wlin = nullptr, *wxc = nullptr, *wgates = nullptr;  // in-projection rows; GDN conv values and gates
+  float *wq = nullptr, *wpart = nullptr;
+  _Float16 *wxh = nullptr, *wgh = nullptr, *whh = nullptr;   // gh: GDN or attention output
   // MTP nextn drafter (blk.N after the N decoder layers; its decoder block
   // is L[n_layers]).  Its KV stream starts at slot 1: slot s lives at index
   // s - 1, *mctl is the last index filled.  Every block commits its
@@ -415,6 +424,117 @@ int block(cwen_model *m, int B, int mode, hipStream_t st) {
   return CWEN_OK;
 }
 
+// ---- prefill: N positions per sweep over the weights.
+
+// Stride of an in-projection row, and whether every matrix takes the wide
+// products.
+int wide_ls(const cwen_model_cfg &c) {
+  const Rows r = rows_of(c);
+  return ((r.lin > r.att ? r.lin : r.att) + 3) / 4 * 4;
+}
+bool wide_model(const cwen_model *m) {
+  if (mtp_ready(m)) return false;      // its commit pass runs per block
+  for (int l = 0; l < m->cfg.n_layers; ++l) {
+    const Layer &y = m->L[l];
+    if (!wide_takes(y.ffn_gu, 2, false) || !wide_takes(y.ffn_down, 1, true) ||
+        !wide_takes(y.linear ? y.lin_in : y.att_in, 1, false) || !wide_takes(y.linear ? y.ssm_out : y.wo, 1, true))
+      return false;
+    if (y.linear && (y.gdn->L || y.gdn->last_B)) return false;
+  }
+  return true;
+}
+
+void wide_free(cwen_model *m) {
+  for (void *p : {(void *)m->wtoks, (void *)m->wX, (void *)m->wssq, (void *)m->wpsc, (void *)m->wlin, (void *)m->wxc,
+                  (void *)m->wgates, (void *)m->wq, (void *)m->wpart, (void *)m->wxh, (void *)m->wgh, (void *)m->whh})
+    if (p) (void)hipFree(p);
+  if (m->hwtok) (void)hipHostFree(m->hwtok);
+  m->wtoks = m->hwtok = nullptr;
+  m->wX = m->wssq = m->wpsc = m->wlin = m->wxc = m->wgates = m->wq = m->wpart = nullptr;
+  m->wxh = m->wgh = m->whh = nullptr;
+  m->wn = 0;
+}
+
+// Workspace for N positions, grown to at most WIDE_MAX.
+int wide_alloc(cwen_model *m, int N) {
+  if (m->wn >= N) return CWEN_OK;
+  wide_free(m);
+  const cwen_model_cfg &c = m->cfg;
+  const Rows R = rows_of(c);
+  const size_t n = (size_t)N, H = c.d_model, Qo = (size_t)R.Qo2 / 2;
+  size_t part = 0;
+  for (int l = 0; l < c.n_layers; ++l) {
+    const Layer &y = m->L[l];
+    part = std::max({part, wide_partial_floats(y.ffn_gu, 2, false, N), wide_partial_floats(y.ffn_down, 1, true, N),
+                     wide_partial_floats(y.linear ? y.lin_in : y.att_in, 1, false, N),
+                     wide_partial_floats(y.linear ? y.ssm_out : y.wo, 1, true, N)});
+  }
+  int rc = (dmalloc(&m->wtoks, n) || dmalloc(&m->wX, n * H) || dmalloc(&m->wssq, n * CWEN_MAX_PARTS) ||
+            dmalloc(&m->wpsc, n + 64) || dmalloc(&m->wlin, n * wide_ls(c)) || dmalloc(&m->wxc, n * R.C) ||
+            dmalloc(&m->wgates, n * 2 * R.nvh) || dmalloc(&m->wq, n * Qo) || dmalloc(&m->wpart, part) ||
+            dmalloc(&m->wxh, n * H) || dmalloc(&m->wgh, n * std::max((size_t)R.Zh, Qo)) ||
+            dmalloc(&m->whh, n * c.d_ffn) ||
+            hipHostMalloc((void **)&m->hwtok, n * sizeof(int), hipHostMallocDefault) != hipSuccess)
+               ? CWEN_ENOMEM
+               : CWEN_OK;
+  if (rc) {
+    wide_free(m);
+    (void)hipGetLastError();   // the caller goes on without the workspace
+  } else {
+    m->wn = N;
+  }
+  return rc;
+}
+
+// The commit of N accepted positions: the history moved by one slot.
+__global__ void wide_advance_kernel(int *ctl, int n, int nslot) {
+  ctl[0] += n;
+  ctl[1] = (ctl[1] + 1) % nslot;
+}
+
+// `block` (MODE_FWD) for N positions, a multiple of 16, tokens in m->wtoks.
+int wide_block(cwen_model *m, int N, hipStream_t st) {
+  const cwen_model_cfg &c = m->cfg;
+  cwen_ctx *ctx = m->ctx;
+  const int H = c.d_model, ls = wide_ls(c);
+  const Rows r = rows_of(c);
+  int *const rflag = m->ctl + 5;
+  int rc;
+  if ((rc = embed_launch(m->emb_qs, m->emb_sc, m->emb_type, m->wtoks, N, H, m->wX, H, m->wssq, st, m->wxh,
+                         m->L[0].attn_norm, rflag)))
+    return rc;
+  int npart = 1;
+  for (int l = 0; l < c.n_layers; ++l) {
+    Layer &y = m->L[l];
+    if ((rc = wide_scale(m->wssq, npart, H, c.rms_eps, N, m->wpsc, st))) return rc;
+    const WideOut oin = {m->wlin, ls, 0, nullptr, nullptr, nullptr, nullptr};
+    if ((rc = wide_gemm(ctx, y.linear ? y.lin_in : y.att_in, GEMV_EPI_STORE, m->wxh, N, m->wpsc, oin, m->wpart, st)))
+      return rc;
+    if (y.linear)
+      rc = gdn_wide_launch(y.gdn, m->wlin, ls, r.C, r.o_alpha, r.o_beta, y.ssm_conv, y.ssm_norm, y.ssm_a, y.ssm_dt,
+                           m->wxc, m->wgates, m->wgh, N, rflag, st);
+    else
+      rc = attention_wide_launch(m->wlin, ls, m->wlin + r.Qo2, m->wlin + r.Qo2 + r.Ko, ls, y.q_norm, y.k_norm, m->wq,
+                                 y.K, y.V, m->ctl, m->pos, N, c.n_head, c.n_kv_head, c.n_rot_pairs, c.n_rot,
+                                 c.rope_theta, c.rms_eps, m->apart, c.max_ctx, m->wgh, st, rflag);
+    if (rc) return rc;
+    const cwen_weight *wout = y.linear ? y.ssm_out : y.wo;
+    const WideOut oo = {m->wX, H, 1, m->wxh, y.post_norm, m->wssq, rflag};
+    if ((rc = wide_gemm(ctx, wout, GEMV_EPI_STORE, m->wgh, N, nullptr, oo, m->wpart, st)) ||
+        (rc = wide_scale(m->wssq, gemv_row_tiles(wout), H, c.rms_eps, N, m->wpsc, st)))
+      return rc;
+    const WideOut of = {nullptr, 0, 0, m->whh, nullptr, nullptr, rflag};
+    const WideOut od = {m->wX, H, 1, m->wxh, l + 1 < c.n_layers ? m->L[l + 1].attn_norm : m->out_norm, m->wssq, rflag};
+    if ((rc = wide_gemm(ctx, y.ffn_gu, GEMV_EPI_SWIGLU, m->wxh, N, m->wpsc, of, m->wpart, st)) ||
+        (rc = wide_gemm(ctx, y.ffn_down, GEMV_EPI_STORE, m->whh, N, nullptr, od, m->wpart, st)))
+      return rc;
+    npart = gemv_row_tiles(y.ffn_down);
+  }
+  hipLaunchKernelGGL(wide_advance_kernel, dim3(1), dim3(1), 0, st, m->ctl, N, CWEN_BMAX + 1);
+  CWEN_HIP_TRY(hipGetLastError());
+  return CWEN_OK;
+}
+
 void drop_graphs(cwen_model *m) {
   for (auto &mode : m->gexec)
     for (auto &row : mode)
@@ -699,6 +819,7 @@ int cwen_model_free(cwen_model *m) {
   (void)hipSetDevice(m->ctx->device);
   (void)hipDeviceSynchronize();
   drop_graphs(m);
+  wide_free(m);
   if (m->cap) (void)hipStreamDestroy(m->cap);
   if (m->tok_ev) (void)hipEventDestroy(m->tok_ev);
   for (int l = 0; m->L && l <= m->cfg.n_layers; ++l) {
@@ -921,6 +1042,38 @@ int cwen_model_forward(cwen_model *m, const int *toks, int B, int want_argmax, i
   }
   commit(m, B, B);
   return want_argmax && m->hres[0] ? CWEN_ERANGE : CWEN_OK;
+}
+
+int cwen_model_prefill(cwen_model *m, const int *toks, int n, void *stream) {
+  if (!m || !toks || n < 0 || n % CWEN_BMAX || !ready(m)) return CWEN_EINVAL;
+  if (m->pos + n >= m->cfg.max_ctx) return CWEN_EINVAL;
+  for (int i = 0; i < n; ++i)
+    if (toks[i] < 0 || toks[i] >= m->cfg.vocab) return CWEN_EINVAL;
+  hipStream_t st = (hipStream_t)stream;
+  int i = 0, rc;
+  // A single block has nothing to share; a device without room for the
+  // workspace takes the blocks as well.
+  if (n > CWEN_BMAX && wide_model(m)) {
+    CWEN_HIP_TRY(hipSetDevice(m->ctx->device));
+    if (wide_alloc(m, n < WIDE_MAX ? n : WIDE_MAX) == CWEN_OK)
+      while (i < n) {
+        const int N = n - i < m->wn ? n - i : m->wn;
+        CWEN_HIP_TRY(hipEventSynchronize(m->tok_ev));
+        memcpy(m->hwtok, toks + i, (size_t)N * sizeof(int));
+        CWEN_HIP_TRY(hipMemcpyAsync(m->wtoks, m->hwtok, (size_t)N * sizeof(int), hipMemcpyHostToDevice, st));
+        CWEN_HIP_TRY(hipEventRecord(m->tok_ev, st));
+        if ((rc = wide_block(m, N, st))) return rc;
+        for (int l = 0; l < m->cfg.n_layers; ++l)
+          if (m->L[l].linear) m->L[l].gdn->cur = (m->L[l].gdn->cur + 1) % m->L[l].gdn->nslot;
+        m->pos += N;
+        i += N;
+      }
+  }
+  for (; i < n; i += CWEN_BMAX) {
+    if ((rc = run_block(m, toks + i, CWEN_BMAX, MODE_FWD, st))) return rc;
+    commit(m, CWEN_BMAX, CWEN_BMAX);
+  }
+  return CWEN_OK;
 }
 
 int cwen_model_verify(cwen_model *m, const int *blk, int B, int *k_out, int *bonus_out, void *stream) {

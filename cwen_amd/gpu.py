@@ -55,6 +55,7 @@ SIGNATURES = [
     ("cwen_model_pos", _I, [_VP]),
     ("cwen_model_capacity", _I, [_VP]),
     ("cwen_model_forward", _I, [_VP, _VP, _I, _I, _VP, _VP]),
+    ("cwen_model_prefill", _I, [_VP, _VP, _I, _VP]),
     ("cwen_model_verify", _I, [_VP, _VP, _I, C.POINTER(_I), C.POINTER(_I), _VP]),
     ("cwen_model_logits", _I, [_VP, _VP, _I]),
     ("cwen_model_has_mtp", _I, [_VP]),
@@ -558,6 +559,11 @@ class Model:
         check("cwen_model_forward", lib().cwen_model_forward(self.h, t.ctypes.data, t.size, int(want_argmax),
                                                              am.ctypes.data if want_argmax else None, None))
         return am if want_argmax else None
+
+    def prefill(self, toks) -> None:
+        """Fill the next positions (a multiple of 16) without a head pass."""
+        t = np.ascontiguousarray(toks, dtype=np.int32)
+        check("cwen_model_prefill", lib().cwen_model_prefill(self.h, t.ctypes.data, t.size, None))
 
     def verify(self, blk) -> tuple[int, int]:
         t = np.ascontiguousarray(blk, dtype=np.int32)

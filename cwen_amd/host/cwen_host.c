@@ -50,7 +50,10 @@ int cwen_prefill(cwen_model *m, const int *prompt, int n_prompt, int *next) {
   if (!m || !prompt || n_prompt < 1 || !next) return CWEN_EINVAL;
   int rc = cwen_model_reset(m);
   if (rc) return rc;
-  for (int i = 0; i < n_prompt;) {
+  /* every whole block but the last in one call, which shares the weight sweeps */
+  int i = (n_prompt - 1) / PREFILL_BLOCK * PREFILL_BLOCK;
+  if (i > 0 && (rc = cwen_model_prefill(m, prompt, i, NULL))) return rc;
+  while (i < n_prompt) {
     int B = n_prompt - i;
     if (B > PREFILL_BLOCK) B = PREFILL_BLOCK;
     const int last = i + B == n_prompt;

@@ -289,6 +289,13 @@ int cwen_model_capacity(const cwen_model *m);
  * of magnitude 65520 or more; without want_argmax the next synchronous call
  * reports it. */
 int cwen_model_forward(cwen_model *m, const int *toks, int B, int want_argmax, int *argmax_out, void *stream);
+/* prefill_forward's blocks without a head (run.c:4823-4857): fill positions
+ * pos+1 .. pos+n with HOST token ids, the state and caches bit for bit those
+ * of forward blocks of 16.  n a multiple of 16.  Where the model allows it
+ * (no MTP block, no accepted prefix pending) up to 1024 positions share one
+ * sweep over the weights, on a workspace allocated at the first such call and
+ * held by the model.  Asynchronous like a headless cwen_model_forward. */
+int cwen_model_prefill(cwen_model *m, const int *toks, int n, void *stream);
 /* One speculative verify cycle on the device: score blk[0..B-1] (blk[0] the
  * pending token, blk[1..B-1] the drafts), take the per-row argmax, walk the
  * drafts (run.c:4954-4956) and keep the accepted prefix: the state advances
