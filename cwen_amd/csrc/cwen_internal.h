@@ -176,6 +176,12 @@ __device__ __forceinline__ float f32_of(float x) {
   return x;
 }
 
+// f16 operand of a product over many positions: 128-K tiles of all N
+// positions, [K / 128][N][128].  A row-major operand would put the same K of
+// every position a row apart, a multiple of 2 KB at every model width: on 1 or
+// 2 of an L2's 16 channels.
+__device__ __forceinline__ size_t wide_at(int c, int k, int N) { return ((size_t)(k >> 7) * N + c) * 128 + (k & 127); }
+
 // Row-tile partials of a column's sum of squares: at most 128 per column.
 constexpr int CWEN_MAX_PARTS = 128;
 
@@ -266,7 +272,7 @@ struct WideOut {
   float *y;          // STORE: f32 result [c*ys + row]
   int ys;
   int accumulate;    // y += result
-  _Float16 *yh;      // SWIGLU: silu(A)*B; STORE (nullable): y * nwh[row]; [c*M + row]
+  _Float16 *yh;      // SWIGLU: silu(A)*B; STORE (nullable): y * nwh[row]; in wide_at's order
   const float *nwh;
   float *ssq;        // STORE, nullable: sums of squares of y per 64 rows [c][CWEN_MAX_PARTS]
   int *rflag;        // set to 1 when an f16 value written is not finite
@@ -280,7 +286,7 @@ size_t wide_partial_floats(const cwen_weight *w, int nsides, bool finish, int N)
 // The per-position scale of a normalised operand (GemvPost) for N positions;
 // psc holds N floats rounded up to a multiple of 64.
 int wide_scale(const float *ssq, int npart, int K, float eps, int N, float *psc, hipStream_t st);
-// epi STORE or SWIGLU; psc nullable.
+// epi STORE or SWIGLU; xh in wide_at's order; psc nullable.
 int wide_gemm(const cwen_ctx *ctx, const cwen_weight *w, int epi, const _Float16 *xh, int N, const float *psc,
               const WideOut &o, float *part, hipStream_t st);
 
@@ -297,6 +303,7 @@ void gdn_conv_out(const cwen_gdn *g, const float *kw, GemvOut &o);
 // N positions (a whole number of 16-position blocks) of a prefill, all
 // accepted: `lin` holds the in-projection's rows [N][ls] (qkv, then z at
 // column zo and the raw gates at ao and bo); its qkv columns are overwritten.
+// outh in wide_at's order.
 // xc [N][C] and gates [N][2][nvh] are scratch.  The layer must have no pending replay; the
 // state advances in place and the history moves to slot cur + 1.
 int gdn_wide_launch(const cwen_gdn *g, float *lin, int ls, int zo, int ao, int bo, const float *kw, const float *wn,
@@ -308,11 +315,12 @@ int gdn_peek_launch(const cwen_gdn *g, int L, int buf, float *S_out, hipStream_t
 
 // ------------------------------------------------------------ model.hip
 // Also writes each row's sum of squares to ssq[b][0] (one partial per column)
-// and, when xh is given, the f16 operand x * nw of the first RMSNorm.
+// and, when xh is given, the f16 operand x * nw of the first RMSNorm (row-major, or
+// with `tiled` in wide_at's order).
 // rflag (nullable) is set to 1 when an f16 value written is not finite.
 int embed_launch(const uint8_t *qs, const uint16_t *sc, int type, const int *toks, int B, int H, float *X,
                  int xs, float *ssq, hipStream_t st, _Float16 *xh = nullptr, const float *nw = nullptr,
-                 int *rflag = nullptr);
+                 int *rflag = nullptr, bool tiled = false);
 size_t attn_partial_floats(int NH, int NKV, int max_ctx, int B);
 int attention_init();
 // Largest query heads per KV head the attention kernels take at every block
@@ -328,7 +336,7 @@ int attention_launch(const float *qfull, int qfs, const float *kx, const float *
                      int npairs, int nrot, float theta, float eps, float *part, int max_ctx, _Float16 *yh,
                      hipStream_t st, int *rflag = nullptr, int last_hint = -1);
 // The same for N positions (a whole number of 16-position blocks): qbuf
-// [N][NH][256], yh [N][NH*256]; `part` as for B = 16; last_host: the host's
+// [N][NH][256], yh in wide_at's order; `part` as for B = 16; last_host: the host's
 // copy of *last.
 int attention_wide_launch(const float *qfull, int qfs, const float *kx, const float *vx, int kvs, const float *qn,
                           const float *kn, float *qbuf, float *K, float *V, const int *last, int last_host, int N, int NH,

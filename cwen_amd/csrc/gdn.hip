@@ -315,7 +315,7 @@ struct GdnWide {
   const float *kw, *wn, *A, *dt;
   float *xc;                          // [N][C]: post-conv, q and k l2-normalised
   float *gates;                       // [N][2][nvh]: g, beta
-  _Float16 *outh;                     // [N][nvh*DK]
+  _Float16 *outh;                     // wide_at order
   int *rflag;
   int nkh, nvh, C, N;
 };
@@ -485,7 +485,7 @@ __global__ __launch_bounds__(256) void gdn_wide_norm_kernel(GdnWide p) {
   r.x = wn2.x * o.x * sc * silu_ref(z0);
   r.y = wn2.y * o.y * sc * silu_ref(z1);
   const half2_t h = {(_Float16)f32_of(r.x), (_Float16)f32_of(r.y)};
-  *(half2_t *)(p.outh + (size_t)b * p.nvh * DK + hv * DK + 2 * lane) = h;
+  *(half2_t *)(p.outh + wide_at(b, hv * DK + 2 * lane, p.N)) = h;
   if (f16_bad(h[0]) || f16_bad(h[1])) raise_flag(p.rflag);
 }
 

@@ -63,7 +63,7 @@ __device__ __forceinline__ void embed_block_q6k(const uint8_t *row, int i, float
 
 __global__ __launch_bounds__(256) void embed_kernel(const uint8_t *qs, const uint16_t *sc, int type,
                                                     const int *toks, int H, float *X, int xs, float *ssq,
-                                                    _Float16 *xh, const float *nw, int *rflag) {
+                                                    _Float16 *xh, const float *nw, int *rflag, int tiled) {
   __shared__ float red[4];
   const int b = blockIdx.x;
   const size_t tok = (size_t)toks[b];
@@ -98,8 +98,9 @@ __global__ __launch_bounds__(256) void embed_kernel(const uint8_t *qs, const uin
       dst[j + 16] = hi;
       if (xh) {
         const _Float16 h0 = (_Float16)(lo * nw[i * 32 + j]), h1 = (_Float16)(hi * nw[i * 32 + j + 16]);
-        xh[(size_t)b * H + i * 32 + j] = h0;
-        xh[(size_t)b * H + i * 32 + j + 16] = h1;
+        _Float16 *xd = xh + (tiled ? wide_at(b, i * 32 + j, (int)gridDim.x) : (size_t)b * H + i * 32 + j);
+        xd[0] = h0;
+        xd[16] = h1;
         if (f16_bad(h0) || f16_bad(h1)) raise_flag(rflag);
       }
       sq = fmaf(lo, lo, sq);
@@ -130,7 +131,8 @@ struct AttnParams {
   float *pm, *pl;      // partial max / sum [NKV][nchunk][B*kvm]
   int nchunk;
   int nbuf;            // chunk buffers in LDS: 2 lands the next chunk during the current one
-  _Float16 *yh;        // gated outputs f16 [B][NH*HD]
+  _Float16 *yh;        // gated outputs f16 [B][NH*HD], or with tiled (total positions) in wide_at's order
+  int tiled;
   int *rflag;          // set to 1 when a gated output is out of f16's range, nullable
 };
 
@@ -447,16 +449,18 @@ __global__ __launch_bounds__(HD * MGR) void attn_merge_kernel(AttnParams p) {
   const float g = p.qfull[(size_t)b * p.qfs + (size_t)h * 2 * HD + HD + d];
   const float y = (O / L) * (1.f / (1.f + expf(-g)));
   const _Float16 yh = (_Float16)y;
-  p.yh[(size_t)b * p.NH * HD + (size_t)h * HD + d] = yh;
+  p.yh[p.tiled ? wide_at(p.off + b, h * HD + d, p.tiled) : (size_t)b * p.NH * HD + (size_t)h * HD + d] = yh;
   if (f16_bad(yh)) raise_flag(p.rflag);
 }
 
 }  // namespace
 
 int embed_launch(const uint8_t *qs, const uint16_t *sc, int type, const int *toks, int B, int H, float *X,
-                 int xs, float *ssq, hipStream_t st, _Float16 *xh, const float *nw, int *rflag) {
+                 int xs, float *ssq, hipStream_t st, _Float16 *xh, const float *nw, int *rflag,
+                 bool tiled) {
   if ((xh == nullptr) != (nw == nullptr)) return CWEN_EINVAL;
-  hipLaunchKernelGGL(embed_kernel, dim3((unsigned)B), dim3(256), 0, st, qs, sc, type, toks, H, X, xs, ssq, xh, nw, rflag);
+  hipLaunchKernelGGL(embed_kernel, dim3((unsigned)B), dim3(256), 0, st, qs, sc, type, toks, H, X, xs, ssq, xh, nw, rflag,
+                     (int)tiled);
   CWEN_HIP_TRY(hipGetLastError());
   return CWEN_OK;
 }
@@ -508,6 +512,7 @@ void attn_params(AttnParams &p, const float *qfull, int qfs, const float *kx, co
   p.pm = part + (size_t)NKV * p.nchunk * nq * HD;
   p.pl = p.pm + (size_t)NKV * p.nchunk * nq;
   p.yh = yh;
+  p.tiled = 0;
   p.rflag = rflag;
 }
 }  // namespace
@@ -552,11 +557,11 @@ int attention_wide_launch(const float *qfull, int qfs, const float *kx, const fl
   attn_params(p, qfull, qfs, kx, vx, kvs, qn, kn, qbuf, K, V, last, B, NH, NKV, npairs, nrot, theta, eps, part, max_ctx,
               yh, rflag);
   hipLaunchKernelGGL(attn_prep_kernel, dim3((unsigned)N, (unsigned)(NH + NKV)), dim3(HD), 0, st, p);
+  p.tiled = N;
   for (int j = 0; j < N; j += B) {
     p.off = j;
     p.q = qbuf + (size_t)j * NH * HD;
     p.qfull = qfull + (size_t)j * qfs;
-    p.yh = yh + (size_t)j * NH * HD;
     const bool wide = attention_wide(last_host + j + B);
     const int wgs = wide ? ATTN_WIDE_WGS : ATTN_NARROW_WGS;
     p.nbuf = wide ? 1 : 2;

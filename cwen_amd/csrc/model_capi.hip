@@ -501,7 +501,7 @@ int wide_block(cwen_model *m, int N, hipStream_t st) {
   int *const rflag = m->ctl + 5;
   int rc;
   if ((rc = embed_launch(m->emb_qs, m->emb_sc, m->emb_type, m->wtoks, N, H, m->wX, H, m->wssq, st, m->wxh,
-                         m->L[0].attn_norm, rflag)))
+                         m->L[0].attn_norm, rflag, true)))
     return rc;
   int npart = 1;
   for (int l = 0; l < c.n_layers; ++l) {

@@ -15,18 +15,19 @@
 //
 // Design (gfx950).  A block of 16 positions re-reads every weight, so a
 // prompt in such blocks is bound by HBM (4096 positions: 256 sweeps).  Here a
-// workgroup of 4 waves takes SPW weight streams of 16 rows per wave and 16 P
-// positions: the quantized bytes go from HBM to registers and are unpacked
-// there, once per 16 P positions; the activations are staged in LDS 128 K at
-// a time (double-buffered, XOR-swizzled as in gemv_kernel), shared by the 4
-// waves.  With SPW = P = 4 a wave issues 64 MFMAs (1024 matrix-core cycles)
-// per 128 K against 224 VALU operations of unpacking (896 cycles) and 16 KB of
-// LDS reads; two workgroups per CU overlap them.  Measured on 4 layers of the
-// 27B shape, 4096 positions: 97.6 ms in blocks of 16, 39.3 ms in four passes
-// of 1024; the gate/up product takes 741 us of a pass, 0.49 PFLOP/s.
-// Workgroups are numbered so that each XCD takes a contiguous range of row
-// blocks with all their positions: the weights cross one XCD's L2 once, the
-// activations stay in every L2.
+// workgroup of 4 waves takes SPW weight streams of 16 rows per wave and 64
+// positions: the quantized bytes go from memory to registers and are unpacked
+// there, once per 64 positions; the activations are staged in LDS 128 K at
+// a time (double-buffered), shared by the 4 waves.  With SPW = 4 a wave issues
+// 64 MFMAs (1024 matrix-core cycles) per 128 K against 224 VALU operations of
+// unpacking (896 cycles) and 16 KB of LDS reads; two workgroups per CU overlap
+// them.  128 accumulator registers per lane leave no room for a second set of
+// operands: with 8 position tiles and one workgroup per CU the compiler spilled
+// loads in flight (739 us for gate/up below), and 8 position tiles of 2 streams,
+// half the unpacking per product, came to the same time as this (395 us).
+// Measured, gate/up 2 x 17408 x 5120 at 1024 positions: 392 us, 0.93 PFLOP/s
+// (a library f16 product of 8192^3 on the same card: 1.18).  4096 positions at
+// 4 layers of the 27B shape: 97.6 ms in blocks of 16, 28.1 ms in passes of 1024.
 #include <algorithm>
 
 #include "cwen_internal.h"
@@ -41,9 +42,9 @@ struct WideParams {
   const uint8_t *w;
   uint32_t wbytes;
   int nrg, nst, M;
-  const _Float16 *xh;                // [N][K]
+  const _Float16 *xh;                // activations, wide_at order
   int K, N, npt;                     // npt: position tiles (16 P positions each)
-  int items;                         // row items x npt
+  int items, perA, perB;             // row items x npt; whole items and pieces per XCD
   // Row items: nA row blocks computed whole, covering row groups [0, rgB);
   // then the row blocks of [rgB, nrg), S pieces of rps rounds each, whose
   // sums go to `part` [piece][side][N][rowsB].
@@ -63,18 +64,20 @@ template <int FMT> struct TileRegs {
 };
 
 template <int FMT, int NS, int EPI, int SPW, int P>
-__global__ __launch_bounds__(64 * WW, 2) void wide_kernel(WideParams p) {
+__global__ __launch_bounds__(64 * WW, P * SPW > 16 ? 1 : 2) void wide_kernel(WideParams p) {
   using F = Fmt<FMT>;
   constexpr int RGW = SPW / NS;      // row groups per wave
   constexpr bool DM = FMT == GEMV_Q41 || FMT == GEMV_Q5K;
   using ScT = std::conditional_t<DM, uint4, uint2>;
   __shared__ uint4 act[2][P * 256];  // [buf][position][unit ^ (position & 15)]
 
-  const int per = (int)gridDim.x >> 3;
-  const int item0 = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
-  if (item0 >= p.items) return;
-  const int pt = item0 % p.npt, item = item0 / p.npt;
-  const bool piece = item >= p.nA;
+  // XCD x (workgroups x, x + 8, ...) takes a contiguous range of the whole
+  // items and one of the pieces, positions fastest.
+  const int x = (int)blockIdx.x & 7, j = (int)blockIdx.x >> 3;
+  const bool piece = j >= p.perA;
+  const int it = piece ? p.nA * p.npt + x * p.perB + j - p.perA : x * p.perA + j;
+  if (it >= (piece ? p.items : p.nA * p.npt)) return;
+  const int pt = it % p.npt, item = it / p.npt;
   const int sp = piece ? (item - p.nA) % p.S : 0;
   const int rb = piece ? (item - p.nA) / p.S : item;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -96,18 +99,22 @@ __global__ __launch_bounds__(64 * WW, 2) void wide_kernel(WideParams p) {
     wofs[s] = (((uint32_t)r0 * p.nrg + rg) * NS + s % NS) * F::ST_BYTES;
   }
 
-  // Activations: thread t stages unit (t & 15) ^ (t >> 4) of positions
-  // (t >> 4) + 16 i; positions past N lie past the buffer range (zeros).
-  uint32_t xofs[P];
-#pragma unroll
-  for (int i = 0; i < P; ++i)
-    xofs[i] = (uint32_t)(pt * 16 * P + 16 * i + (tid >> 4)) * (uint32_t)(p.K * 2) + ((tid & 15) ^ (tid >> 4)) * 16 +
-              (uint32_t)r0 * (Q4_ST_K * 2);
+  // Activations: thread t stages LDS unit t & 15 of positions
+  // (t >> 4) + 16 i of the tile's positions, 256 contiguous bytes each; those
+  // past N read the next tile's first positions, or zeros past the buffer:
+  // their sums are never stored.
+  // LDS unit of K unit u of position c: c * 16 + (u' ^ (c & 15)), u' = u with
+  // its upper two bits negated.  A 16-byte LDS read serves 16 lanes at a time,
+  // lanes 0-3, 12-15, 20-23 and 24-27 first: with this order they meet 16
+  // different units (u ^ c gave a 2-way conflict on every operand read).
+  const int xu = (tid & 15) ^ (tid >> 4);
+  const uint32_t xofs = (uint32_t)(pt * 16 * P + (tid >> 4)) * 256 + ((((4 - (xu >> 2)) & 3) << 2) | (xu & 3)) * 16;
+  const uint32_t xtile = (uint32_t)p.N * 256, xof0 = (uint32_t)r0 * 4 * xtile;
   uint4 xa[P];
   auto act_load = [&](int t) __attribute__((always_inline)) {
-    const uint32_t so = (uint32_t)min(t, ntile - 1) * (Q4_TILE_K * 2);
+    const uint32_t so = xof0 + (uint32_t)min(t, ntile - 1) * xtile;
 #pragma unroll
-    for (int i = 0; i < P; ++i) xa[i] = bload16(xr, xofs[i], so);
+    for (int i = 0; i < P; ++i) xa[i] = bload16(xr, xofs + i * 4096, so);
   };
   auto act_store = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -122,14 +129,14 @@ __global__ __launch_bounds__(64 * WW, 2) void wide_kernel(WideParams p) {
     for (int s = 0; s < SPW; ++s) {
 #pragma unroll
       for (int v = 0; v < F::TV; ++v)
-        wq[b][s].q[v] = bload16_nt(wr, lane * 16 + v * 1024, wofs[s] + so + u * (1024 * F::TV));
+        wq[b][s].q[v] = bload16(wr, lane * 16 + v * 1024, wofs[s] + so + u * (1024 * F::TV));
       if constexpr (FMT == GEMV_Q6K)
         wq[b][s].hi = bload8_nt(wr, lane * 16, wofs[s] + so + F::HI_OFS + (u >> 1) * 1024 + (u & 1) * 8);
       if constexpr (FMT == GEMV_Q5K) wq[b][s].hi.x = bload4_nt(wr, lane * 16, wofs[s] + so + F::HI_OFS + u * 4);
     }
   };
-  ScT sc[SPW], scn[SPW];
-  uint32_t dq[SPW] = {}, dqn[SPW] = {};
+  ScT sc[SPW];
+  uint32_t dq[SPW] = {};
   auto sc_load = [&](ScT (&d)[SPW], uint32_t (&dd)[SPW], int r) __attribute__((always_inline)) {
     const uint32_t so = (uint32_t)min(r, nround - 1) * sstride;
 #pragma unroll
@@ -148,7 +155,47 @@ __global__ __launch_bounds__(64 * WW, 2) void wide_kernel(WideParams p) {
   const Unpack uc = unpack_consts();
   int aslot[4];
 #pragma unroll
-  for (int m = 0; m < 4; ++m) aslot[m] = n * 16 + ((4 * g + m) ^ n);
+  for (int m = 0; m < 4; ++m) aslot[m] = n * 16 + ((4 * ((4 - g) & 3) + m) ^ n);
+
+  // Scales of tile u of the round (Q4_1 / Q5_K: scale, offset; Q6_K: per half
+  // block).
+  half2_t d0[SPW], d1[SPW];
+  auto scales = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < SPW; ++s) {
+      if constexpr (FMT == GEMV_Q6K) {
+        const half2_t s2 = i8pair(u < 2 ? sc[s].x : sc[s].y, uc.magic, u & 1);
+        const half2_t ds = s2 * bcast_half(dq[s], u >= 2);
+        d0[s] = (half2_t){ds[0], ds[0]};
+        d1[s] = (half2_t){ds[1], ds[1]};
+      } else if constexpr (DM) {
+        const uint32_t w = u == 0 ? sc[s].x : u == 1 ? sc[s].y : u == 2 ? sc[s].z : sc[s].w;
+        d0[s] = bcast_half(w, false);
+        d1[s] = bcast_half(w, true);
+      } else {
+        d0[s] = d1[s] = bcast_half(u < 2 ? sc[s].x : sc[s].y, (u & 1) != 0);
+      }
+    }
+  };
+  // MFMA operand of K run m of stream s, from tile buffer tb.
+  auto operand = [&](int tb, int m, int s) __attribute__((always_inline)) -> half8_t {
+    const TileRegs<FMT> &w = wq[tb][s];
+    const uint32_t qm = m == 0 ? w.q[0].x : m == 1 ? w.q[0].y : m == 2 ? w.q[0].z : w.q[0].w;
+    if constexpr (FMT == GEMV_Q4) {
+      return unpack8_q4(qm, uc, d0[s]);
+    } else if constexpr (FMT == GEMV_Q41) {
+      return unpack8_q41(qm, uc, d0[s], d1[s]);
+    } else if constexpr (FMT == GEMV_Q5K) {
+      const uint32_t h = w.hi.x;
+      return unpack8_q5(qm, h >> m, h >> (8 + m), h << (8 - m), uc, d0[s], d1[s]);
+    } else if constexpr (FMT == GEMV_Q6K) {
+      const uint32_t h = m < 2 ? w.hi.x : w.hi.y;
+      return unpack8_q6(qm, (m & 1) ? rotl8(h) : h, uc, m < 2 ? d0[s] : d1[s]);
+    } else {
+      const uint4 &q = w.q[m >> 1];
+      return (m & 1) ? unpack8_q8(q.z, q.w, uc.magic, d0[s]) : unpack8_q8(q.x, q.y, uc.magic, d0[s]);
+    }
+  };
 
   act_load(0);
   sc_load(sc, dq, 0);
@@ -157,66 +204,35 @@ __global__ __launch_bounds__(64 * WW, 2) void wide_kernel(WideParams p) {
   act_load(1);
   lds_barrier();
 
+  // One 128-K tile per step.  The scheduling barriers keep the request order
+  // (activations of tile t + 2, weights of tile t + 1) and one K run's operands
+  // live at a time: without them the scheduler hoists reads until it spills.
   for (int r = 0; r < nround; ++r) {
-    sc_load(scn, dqn, r + 1);
 #pragma unroll
     for (int u = 0; u < Q4_ST_TILES; ++u) {
       const int t = r * Q4_ST_TILES + u;
       act_store((u + 1) & 1);          // tile t + 1 (its buffer's readers passed the last barrier)
+      __builtin_amdgcn_sched_barrier(0);
       act_load(t + 2);
       tile_load((u + 1) & 1, t + 1);
-      half2_t d0[SPW], d1[SPW];        // scales of the tile (Q4_1 / Q5_K: scale, offset; Q6_K: per half block)
-#pragma unroll
-      for (int s = 0; s < SPW; ++s) {
-        if constexpr (FMT == GEMV_Q6K) {
-          const half2_t s2 = i8pair(u < 2 ? sc[s].x : sc[s].y, uc.magic, u & 1);
-          const half2_t ds = s2 * bcast_half(dq[s], u >= 2);
-          d0[s] = (half2_t){ds[0], ds[0]};
-          d1[s] = (half2_t){ds[1], ds[1]};
-        } else if constexpr (DM) {
-          const uint32_t w = u == 0 ? sc[s].x : u == 1 ? sc[s].y : u == 2 ? sc[s].z : sc[s].w;
-          d0[s] = bcast_half(w, false);
-          d1[s] = bcast_half(w, true);
-        } else {
-          d0[s] = d1[s] = bcast_half(u < 2 ? sc[s].x : sc[s].y, (u & 1) != 0);
-        }
-      }
-      const uint4 *A = act[u & 1];
+      scales(u);
+      if (u == 3) sc_load(sc, dq, r + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         half8_t a[P];
 #pragma unroll
-        for (int i = 0; i < P; ++i) a[i] = __builtin_bit_cast(half8_t, A[aslot[m] + 256 * i]);
+        for (int i = 0; i < P; ++i) a[i] = __builtin_bit_cast(half8_t, act[u & 1][aslot[m] + 256 * i]);
 #pragma unroll
         for (int s = 0; s < SPW; ++s) {
-          const TileRegs<FMT> &w = wq[u & 1][s];
-          const uint32_t qm = m == 0 ? w.q[0].x : m == 1 ? w.q[0].y : m == 2 ? w.q[0].z : w.q[0].w;
-          half8_t b;
-          if constexpr (FMT == GEMV_Q4) {
-            b = unpack8_q4(qm, uc, d0[s]);
-          } else if constexpr (FMT == GEMV_Q41) {
-            b = unpack8_q41(qm, uc, d0[s], d1[s]);
-          } else if constexpr (FMT == GEMV_Q5K) {
-            const uint32_t h = w.hi.x;
-            b = unpack8_q5(qm, h >> m, h >> (8 + m), h << (8 - m), uc, d0[s], d1[s]);
-          } else if constexpr (FMT == GEMV_Q6K) {
-            const uint32_t h = m < 2 ? w.hi.x : w.hi.y;
-            b = unpack8_q6(qm, (m & 1) ? rotl8(h) : h, uc, m < 2 ? d0[s] : d1[s]);
-          } else {
-            const uint4 &q = w.q[m >> 1];
-            b = (m & 1) ? unpack8_q8(q.z, q.w, uc.magic, d0[s]) : unpack8_q8(q.x, q.y, uc.magic, d0[s]);
-          }
+          const half8_t b = operand(u & 1, m, s);
 #pragma unroll
           for (int i = 0; i < P; ++i)
             acc[i][s][m & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b, acc[i][s][m & 1], 0, 0, 0);
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
       lds_barrier();
-    }
-#pragma unroll
-    for (int s = 0; s < SPW; ++s) {
-      sc[s] = scn[s];
-      dq[s] = dqn[s];
     }
   }
 
@@ -249,7 +265,7 @@ __global__ __launch_bounds__(64 * WW, 2) void wide_kernel(WideParams p) {
         for (int d = 0; d < NS; ++d) o[d] = p.psc ? v[d][e] * scl[e] : v[d][e];
         if constexpr (EPI == GEMV_EPI_SWIGLU) {
           const _Float16 h = (_Float16)f32_of(silu_f(o[0]) * o[NS - 1]);
-          p.yh[(size_t)c * p.M + row] = h;
+          p.yh[wide_at(c, row, p.N)] = h;
           bad |= f16_bad(h);
         } else {
           p.y[(size_t)c * p.ys + row] = o[0];
@@ -279,7 +295,7 @@ __global__ __launch_bounds__(256) void wide_finish_kernel(WideParams p, WideOut 
   if constexpr (EPI == GEMV_EPI_SWIGLU) {
     if (!ok) return;
     const _Float16 h = (_Float16)f32_of(silu_f(v[0]) * v[NS - 1]);
-    p.yh[(size_t)c * p.M + row] = h;
+    p.yh[wide_at(c, row, p.N)] = h;
     if (f16_bad(h)) raise_flag(p.rflag);
   } else {
     float r = v[0], sq = 0.f;
@@ -288,7 +304,7 @@ __global__ __launch_bounds__(256) void wide_finish_kernel(WideParams p, WideOut 
       p.y[(size_t)c * p.ys + row] = r;
       if (o.yh) {
         const _Float16 h = (_Float16)f32_of(r * o.nwh[row]);
-        o.yh[(size_t)c * p.M + row] = h;
+        o.yh[wide_at(c, row, p.N)] = h;
         if (f16_bad(h)) raise_flag(p.rflag);
       }
       sq = r * r;
@@ -318,7 +334,9 @@ void launch(WideParams p, hipStream_t st) {
   p.npt = (p.N + 16 * P - 1) / (16 * P);
   p.nA = (p.rgB + RGB - 1) / RGB;
   p.items = (p.nA + (p.nrg - p.rgB + RGB - 1) / RGB * p.S) * p.npt;
-  hipLaunchKernelGGL((wide_kernel<FMT, NS, EPI, SPW, P>), dim3((unsigned)((p.items + 7) / 8 * 8)), dim3(64 * WW), 0, st, p);
+  p.perA = (p.nA * p.npt + 7) / 8;
+  p.perB = (p.items - p.nA * p.npt + 7) / 8;
+  hipLaunchKernelGGL((wide_kernel<FMT, NS, EPI, SPW, P>), dim3((unsigned)(8 * (p.perA + p.perB))), dim3(64 * WW), 0, st, p);
 }
 
 }  // namespace
