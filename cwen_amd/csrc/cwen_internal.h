@@ -168,12 +168,19 @@ __device__ __forceinline__ void raise_flag(int *flag) {
   if (flag) __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// A product as f32, so that a conversion after it rounds a second time: the
-// compiler otherwise may fold the two into one mixed-precision operation
-// (v_fma_mixlo_f16), in one kernel and not in another.
+// A product as an f16 operand.  The compiler may fold the product and the
+// conversion into one mixed-precision operation (one rounding) in one kernel
+// and not in another; where two kernels must give the same bits, the form is
+// written out: f32_of keeps the f32 rounding before the conversion,
+// f16_mul rounds once.
 __device__ __forceinline__ float f32_of(float x) {
   asm("" : "+v"(x));
   return x;
+}
+__device__ __forceinline__ _Float16 f16_mul(float a, float b) {
+  uint32_t r;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
+  return __builtin_bit_cast(_Float16, (uint16_t)r);
 }
 
 // f16 operand of a product over many positions: 128-K tiles of all N
@@ -335,13 +342,14 @@ int attention_launch(const float *qfull, int qfs, const float *kx, const float *
                      const float *kn, float *qbuf, float *K, float *V, const int *last, int B, int NH, int NKV,
                      int npairs, int nrot, float theta, float eps, float *part, int max_ctx, _Float16 *yh,
                      hipStream_t st, int *rflag = nullptr, int last_hint = -1);
-// The same for N positions (a whole number of 16-position blocks): qbuf
-// [N][NH][256], yh in wide_at's order; `part` as for B = 16; last_host: the host's
-// copy of *last.
+// The same for N positions: qbuf [N][NH][256], yh in wide_at's order;
+// last_host: the host's copy of *last; part: attention_wide_floats(NH, NKV,
+// last_host + 1 + N, N) floats.
+size_t attention_wide_floats(int NH, int NKV, int ctx_end, int N);
 int attention_wide_launch(const float *qfull, int qfs, const float *kx, const float *vx, int kvs, const float *qn,
                           const float *kn, float *qbuf, float *K, float *V, const int *last, int last_host, int N, int NH,
-                          int NKV, int npairs, int nrot, float theta, float eps, float *part, int max_ctx, _Float16 *yh,
-                          hipStream_t st, int *rflag);
+                          int NKV, int npairs, int nrot, float theta, float eps, float *part, size_t part_floats,
+                          int max_ctx, _Float16 *yh, hipStream_t st, int *rflag);
 // Whether a block whose last position is last_pos takes the wide chunk grid
 // (attention_launch's last_hint; -1 = not known, narrow).  Only the launch
 // shape depends on it, never the result.

@@ -83,7 +83,8 @@ struct cwen_model {
   int *wtoks = nullptr, *hwtok = nullptr;              // device / pinned host tokens
   float *wX = nullptr, *wssq = nullptr, *wpsc = nullptr;
   float *wlin = nullptr, *wxc = nullptr, *wgates = nullptr;  // in-projection rows; GDN conv values and gates
-  float *wq = nullptr, *wpart = nullptr;
+  float *wq = nullptr, *wpart = nullptr, *watt = nullptr;    // watt: the attention's scores and sums
+  size_t watt_floats = 0;
   _Float16 *wxh = nullptr, *wgh = nullptr, *whh = nullptr;   // gh: GDN or attention output
   // MTP nextn drafter (blk.N after the N decoder layers; its decoder block
   // is L[n_layers]).  Its KV stream starts at slot 1: slot s lives at index
@@ -446,22 +447,33 @@ bool wide_model(const cwen_model *m) {
 
 void wide_free(cwen_model *m) {
   for (void *p : {(void *)m->wtoks, (void *)m->wX, (void *)m->wssq, (void *)m->wpsc, (void *)m->wlin, (void *)m->wxc,
-                  (void *)m->wgates, (void *)m->wq, (void *)m->wpart, (void *)m->wxh, (void *)m->wgh, (void *)m->whh})
+                  (void *)m->wgates, (void *)m->wq, (void *)m->wpart, (void *)m->watt, (void *)m->wxh, (void *)m->wgh, (void *)m->whh})
     if (p) (void)hipFree(p);
   if (m->hwtok) (void)hipHostFree(m->hwtok);
   m->wtoks = m->hwtok = nullptr;
-  m->wX = m->wssq = m->wpsc = m->wlin = m->wxc = m->wgates = m->wq = m->wpart = nullptr;
+  m->wX = m->wssq = m->wpsc = m->wlin = m->wxc = m->wgates = m->wq = m->wpart = m->watt = nullptr;
+  m->watt_floats = 0;
   m->wxh = m->wgh = m->whh = nullptr;
   m->wn = 0;
 }
 
-// Workspace for N positions, grown to at most WIDE_MAX.
-int wide_alloc(cwen_model *m, int N) {
-  if (m->wn >= N) return CWEN_OK;
-  wide_free(m);
+// Workspace for the passes over n positions: their length grows to at most
+// WIDE_MAX, the attention's part with the context (bounded, see
+// attention_wide_floats).
+int wide_alloc(cwen_model *m, int n) {
   const cwen_model_cfg &c = m->cfg;
+  int N = std::min(n, WIDE_MAX);
+  size_t att = 0;
+  for (int i = 0; i < n; i += WIDE_MAX) {
+    const int k = std::min(n - i, WIDE_MAX);
+    att = std::max(att, attention_wide_floats(c.n_head, c.n_kv_head, m->pos + 1 + i + k, k));
+  }
+  if (m->wn >= N && m->watt_floats >= att) return CWEN_OK;
+  N = std::max(N, m->wn);
+  att = std::max(att, m->watt_floats);
+  wide_free(m);
   const Rows R = rows_of(c);
-  const size_t n = (size_t)N, H = c.d_model, Qo = (size_t)R.Qo2 / 2;
+  const size_t np = (size_t)N, H = c.d_model, Qo = (size_t)R.Qo2 / 2;
   size_t part = 0;
   for (int l = 0; l < c.n_layers; ++l) {
     const Layer &y = m->L[l];
@@ -469,12 +481,13 @@ int wide_alloc(cwen_model *m, int N) {
                      wide_partial_floats(y.linear ? y.lin_in : y.att_in, 1, false, N),
                      wide_partial_floats(y.linear ? y.ssm_out : y.wo, 1, true, N)});
   }
-  int rc = (dmalloc(&m->wtoks, n) || dmalloc(&m->wX, n * H) || dmalloc(&m->wssq, n * CWEN_MAX_PARTS) ||
-            dmalloc(&m->wpsc, n + 64) || dmalloc(&m->wlin, n * wide_ls(c)) || dmalloc(&m->wxc, n * R.C) ||
-            dmalloc(&m->wgates, n * 2 * R.nvh) || dmalloc(&m->wq, n * Qo) || dmalloc(&m->wpart, part) ||
-            dmalloc(&m->wxh, n * H) || dmalloc(&m->wgh, n * std::max((size_t)R.Zh, Qo)) ||
-            dmalloc(&m->whh, n * c.d_ffn) ||
-            hipHostMalloc((void **)&m->hwtok, n * sizeof(int), hipHostMallocDefault) != hipSuccess)
+  int rc = (dmalloc(&m->wtoks, np) || dmalloc(&m->wX, np * H) || dmalloc(&m->wssq, np * CWEN_MAX_PARTS) ||
+            dmalloc(&m->wpsc, np + 64) || dmalloc(&m->wlin, np * wide_ls(c)) || dmalloc(&m->wxc, np * R.C) ||
+            dmalloc(&m->wgates, np * 2 * R.nvh) || dmalloc(&m->wq, np * Qo) || dmalloc(&m->wpart, part) ||
+            dmalloc(&m->watt, att) ||
+            dmalloc(&m->wxh, np * H) || dmalloc(&m->wgh, np * std::max((size_t)R.Zh, Qo)) ||
+            dmalloc(&m->whh, np * c.d_ffn) ||
+            hipHostMalloc((void **)&m->hwtok, np * sizeof(int), hipHostMallocDefault) != hipSuccess)
                ? CWEN_ENOMEM
                : CWEN_OK;
   if (rc) {
@@ -482,6 +495,7 @@ int wide_alloc(cwen_model *m, int N) {
     (void)hipGetLastError();   // the caller goes on without the workspace
   } else {
     m->wn = N;
+    m->watt_floats = att;
   }
   return rc;
 }
@@ -516,7 +530,7 @@ int wide_block(cwen_model *m, int N, hipStream_t st) {
     else
       rc = attention_wide_launch(m->wlin, ls, m->wlin + r.Qo2, m->wlin + r.Qo2 + r.Ko, ls, y.q_norm, y.k_norm, m->wq,
                                  y.K, y.V, m->ctl, m->pos, N, c.n_head, c.n_kv_head, c.n_rot_pairs, c.n_rot,
-                                 c.rope_theta, c.rms_eps, m->apart, c.max_ctx, m->wgh, st, rflag);
+                                 c.rope_theta, c.rms_eps, m->watt, m->watt_floats, c.max_ctx, m->wgh, st, rflag);
     if (rc) return rc;
     const cwen_weight *wout = y.linear ? y.ssm_out : y.wo;
     const WideOut oo = {m->wX, H, 1, m->wxh, y.post_norm, m->wssq, rflag};
@@ -1055,9 +1069,9 @@ int cwen_model_prefill(cwen_model *m, const int *toks, int n, void *stream) {
   // workspace takes the blocks as well.
   if (n > CWEN_BMAX && wide_model(m)) {
     CWEN_HIP_TRY(hipSetDevice(m->ctx->device));
-    if (wide_alloc(m, n < WIDE_MAX ? n : WIDE_MAX) == CWEN_OK)
+    if (wide_alloc(m, n) == CWEN_OK)
       while (i < n) {
-        const int N = n - i < m->wn ? n - i : m->wn;
+        const int N = std::min(n - i, WIDE_MAX);
         CWEN_HIP_TRY(hipEventSynchronize(m->tok_ev));
         memcpy(m->hwtok, toks + i, (size_t)N * sizeof(int));
         CWEN_HIP_TRY(hipMemcpyAsync(m->wtoks, m->hwtok, (size_t)N * sizeof(int), hipMemcpyHostToDevice, st));

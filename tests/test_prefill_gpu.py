@@ -22,6 +22,8 @@ SMALL = dict(n_layers=4, d_model=1024, d_ffn=2048, vocab=4096, n_head=4, n_kv_he
 # 32-position tiles against 16-query attention groups of 6 heads; q/k/v heads as at the 27B shape
 WIDE = dict(SMALL, d_model=5120, d_ffn=17408, vocab=2048, n_head=24, n_kv_head=4, gdn_nkh=16, gdn_nvh=48)
 ODD = dict(SMALL, d_model=1536, d_ffn=1024, n_head=6, n_kv_head=1, gdn_nkh=4, gdn_nvh=12, full_interval=2)
+# a context at which the attention's scores are made in several batches
+LONG = dict(SMALL, n_layers=2, d_model=512, d_ffn=512, n_head=24, n_kv_head=4, full_interval=2, max_ctx=6400)
 
 
 @pytest.fixture(scope="module")
@@ -54,31 +56,38 @@ def _same(a, b, what):
         assert np.array_equal(x, y), (what, i, float(np.abs(x.astype(np.float64) - y).max()))
 
 
-def _compare(gpu, m, cfg, n, n2=0):
-    toks = synth.rng(9, n).integers(0, cfg["vocab"], n + n2 + 32).astype(np.int32)
+def _compare(gpu, m, cfg, n, n2=0, ragged=0):
+    """n2: positions of a second prompt part; ragged: positions between the
+    two, so that the second starts off any 16 or 32."""
+    toks = synth.rng(9, n).integers(0, cfg["vocab"], n + ragged + n2 + 32).astype(np.int32)
     got = {}
     for how in ("blocks", "prefill"):
         m.reset()
-        for a, b in ((0, n), (n, n + n2)):
-            if how == "prefill":
+        for a, b in ((0, n), (n, n + ragged), (n + ragged, n + ragged + n2)):
+            if b - a == ragged:
+                if ragged:
+                    m.forward(toks[a:b], want_argmax=False)
+            elif how == "prefill":
                 m.prefill(toks[a:b])
             else:
                 for i in range(a, b, 16):
                     m.forward(toks[i:i + 16], want_argmax=False)
             assert m.pos == b - 1
-        got[how] = _after(m, cfg, toks[n + n2:])
+        got[how] = _after(m, cfg, toks[n + ragged + n2:])
     _same(got["prefill"], got["blocks"], (n, n2))
 
 
 @pytest.mark.parametrize("name,n,n2", [("small", 32, 0), ("small", 48, 160), ("small", 1056, 32), ("odd", 80, 0),
-                                       ("odd", 1024, 64), ("wide", 32, 0), ("wide", 336, 48)])
+                                       ("odd", 1024, 64), ("wide", 32, 0), ("wide", 336, 48), ("long", 6144, 80)])
 def test_prefill_equals_blocks(gpu, name, n, n2):
-    cfg = {"small": SMALL, "odd": ODD, "wide": WIDE}[name]
+    cfg = {"small": SMALL, "odd": ODD, "wide": WIDE, "long": LONG}[name]
     print(f"prefill {name}: {n} + {n2} positions", flush=True)
     ctx = gpu.Context(0)
     m = gpu.Model(ctx, **cfg)
     m.synth(3)
     _compare(gpu, m, cfg, n, n2)
+    if n2:
+        _compare(gpu, m, cfg, n, n2, ragged=5)
     m.free()
 
 
