@@ -384,91 +384,102 @@ __global__ __launch_bounds__(256) void gdn_wide_conv_kernel(GdnWide p) {
   }
 }
 
-// The recurrence over N positions: workgroup (slice, head) = 4 waves, wave w
-// columns slice*32 + 8w .. +7 of the head; a lane owns 8 rows x 2 columns of S
-// in registers (rows as in gdn_rec_kernel, so a column's sums have its order).
-// Bound by the chain of one position (decay, 8 FMAs, 4 DPP adds, update);
-// 192 workgroups at 48 heads put one wave on each SIMD of 192 CUs.  The next
-// 16 positions' inputs are requested while 16 are computed; outputs meet in
-// LDS and leave 32 columns at a time, over the row's qkv columns.
+// The recurrence over N positions: workgroup (slice, head) = 8 waves, wave w
+// columns slice*32 + 4w .. +3 of the head; a lane owns 8 rows of one column
+// of S in registers (rows as in gdn_rec_kernel, so a column's sums have its
+// order).  Bound by the chain of one position (decay, 8 FMAs, 4 DPP adds, update)
+// and by issue: 192 workgroups at 48 heads put two waves on each SIMD of 192
+// CUs, so that one's LDS reads and DPP waits pass under the other's FMAs.  With
+// 2 columns per lane and one wave per SIMD, 1024 positions took 310-336 us (a
+// lone wave issues one instruction of any kind per 4 cycles); here 245 us.  The
+// next 16 positions' inputs are requested while 16 are computed; outputs meet
+// in LDS and leave 32 columns at a time, over the row's qkv columns.
 constexpr int WCOLS = 32;            // columns of a head per workgroup
-__global__ __launch_bounds__(256) void gdn_wide_rec_kernel(GdnWide p) {
+__global__ __launch_bounds__(512) void gdn_wide_rec_kernel(GdnWide p) {
+  // q | k per position, each as rows 0-3 of every 8, then rows 4-7: a lane's
+  // two 16-byte reads then meet no bank conflict.
   __shared__ __align__(16) float qk[2][MAXB][2 * DK];
   __shared__ __align__(16) float vs[2][MAXB][WCOLS];
-  __shared__ __align__(16) float ob[MAXB][WCOLS];
-  __shared__ float s_gb[2][2][MAXB];
+  __shared__ __align__(16) float ob[2][MAXB][WCOLS];
+  __shared__ float2 s_gb[2][MAXB];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int slice = blockIdx.x, hv = blockIdx.y, hk = hv % p.nkh;
-  const int rg = lane & 15, cg = lane >> 4;
-  const int i0 = rg * 8, jl = wave * 8 + cg * 2, j0 = slice * WCOLS + jl;
-  float2 s[8];
+  const int rg = lane & 15, i0 = rg * 8;
+  const int jl = wave * 4 + (lane >> 4), j0 = slice * WCOLS + jl;
+  float s[8];
   {
     const float *Sh = p.S_in + (size_t)hv * DK * DK;
 #pragma unroll
-    for (int r = 0; r < 8; ++r) s[r] = *(const float2 *)(Sh + (size_t)(i0 + r) * DK + j0);
+    for (int r = 0; r < 8; ++r) s[r] = Sh[(size_t)(i0 + r) * DK + j0];
   }
   // Staging of 16 positions: thread t loads 4 floats of q|k of positions
-  // (t >> 6) + 4 i, 2 floats of v of position t >> 4, and one gate (t < 32).
-  float4 rq[4];
-  float2 rv;
-  float rgt = 0.f;
+  // t / 64 and t / 64 + 8, one float of v, and (t < 16) a position's gates.
+  float4 rq[2];
+  float rv;
+  float2 rgt = {0.f, 0.f};
+  const int e0 = (tid & 63) * 4, off = e0 < DK ? hk * DK + e0 : (p.nkh + hk) * DK + e0 - DK;
+  const int el = (e0 & DK) + ((e0 >> 2) & 1) * (DK / 2) + ((e0 & (DK - 1)) >> 3) * 4;   // its place in LDS
   auto request = [&](int b0) {
-    const int e = (tid & 63) * 4;
-    const int off = e < DK ? hk * DK + e : (p.nkh + hk) * DK + e - DK;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) rq[i] = *(const float4 *)(p.xc + (size_t)(b0 + (tid >> 6) + 4 * i) * p.C + off);
-    rv = *(const float2 *)(p.xc + (size_t)(b0 + (tid >> 4)) * p.C + 2 * p.nkh * DK + hv * DK + slice * WCOLS + (tid & 15) * 2);
-    if (tid < 32) rgt = p.gates[((size_t)(b0 + (tid & 15)) * 2 + (tid >> 4)) * p.nvh + hv];
+    for (int i = 0; i < 2; ++i) rq[i] = *(const float4 *)(p.xc + (size_t)(b0 + (tid >> 6) + 8 * i) * p.C + off);
+    rv = p.xc[(size_t)(b0 + (tid >> 5)) * p.C + 2 * p.nkh * DK + hv * DK + slice * WCOLS + (tid & 31)];
+    if (tid < MAXB) {
+      rgt.x = p.gates[((size_t)(b0 + tid) * 2 + 0) * p.nvh + hv];
+      rgt.y = p.gates[((size_t)(b0 + tid) * 2 + 1) * p.nvh + hv];
+    }
   };
   auto land = [&](int bf) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *(float4 *)&qk[bf][(tid >> 6) + 4 * i][(tid & 63) * 4] = rq[i];
-    *(float2 *)&vs[bf][tid >> 4][(tid & 15) * 2] = rv;
-    if (tid < 32) s_gb[bf][tid >> 4][tid & 15] = rgt;
+    for (int i = 0; i < 2; ++i) *(float4 *)&qk[bf][(tid >> 6) + 8 * i][el] = rq[i];
+    vs[bf][tid >> 5][tid & 31] = rv;
+    if (tid < MAXB) s_gb[bf][tid] = rgt;
   };
   request(0);
   land(0);
-  __syncthreads();
+  lds_barrier();
   const float scale = 1.f / sqrtf((float)DK);
   for (int b0 = 0, bf = 0; b0 < p.N; b0 += MAXB, bf ^= 1) {
     const bool more = b0 + MAXB < p.N;
     if (more) request(b0 + MAXB);
-#pragma unroll 2
-    for (int b = 0; b < MAXB; ++b) {
-      const float g = s_gb[bf][0][b], beta = s_gb[bf][1][b];
-      const float4 qa = *(const float4 *)&qk[bf][b][i0], qb = *(const float4 *)&qk[bf][b][i0 + 4];
-      const float4 ka = *(const float4 *)&qk[bf][b][DK + i0], kb = *(const float4 *)&qk[bf][b][DK + i0 + 4];
-      const float kr[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
-      const float qr[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
-      const float2 v2 = *(const float2 *)&vs[bf][b][jl];
-      float2 sk = {0.f, 0.f};
+    // No branch between the 8 positions of a half, so that one position's
+    // output sum is scheduled into the next one's chain.
+    auto half = [&](int b8) __attribute__((always_inline)) {
 #pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        s[r].x *= g; s[r].y *= g;
-        sk.x = fmaf(s[r].x, kr[r], sk.x); sk.y = fmaf(s[r].y, kr[r], sk.y);
-      }
-      sk = (float2){sum16(sk.x), sum16(sk.y)};
-      const float2 dl = {beta * (v2.x - sk.x), beta * (v2.y - sk.y)};
-      float2 o = {0.f, 0.f};
+      for (int b = b8; b < b8 + MAXB / 2; ++b) {
+        const float2 gb = s_gb[bf][b];
+        const float g = gb.x, beta = gb.y, v = vs[bf][b][jl];
+        const float4 ka = *(const float4 *)&qk[bf][b][DK + rg * 4], kb = *(const float4 *)&qk[bf][b][DK + DK / 2 + rg * 4];
+        const float4 qa = *(const float4 *)&qk[bf][b][rg * 4], qb = *(const float4 *)&qk[bf][b][DK / 2 + rg * 4];
+        const float kr[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
+        const float qr[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+        float sk = 0.f;
 #pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        s[r].x = fmaf(kr[r], dl.x, s[r].x); s[r].y = fmaf(kr[r], dl.y, s[r].y);
-        o.x = fmaf(s[r].x, qr[r], o.x); o.y = fmaf(s[r].y, qr[r], o.y);
+        for (int r = 0; r < 8; ++r) {
+          s[r] *= g;
+          sk = fmaf(s[r], kr[r], sk);
+        }
+        sk = sum16(sk);
+        const float dl = beta * (v - sk);
+        float o = 0.f;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          s[r] = fmaf(kr[r], dl, s[r]);
+          o = fmaf(s[r], qr[r], o);
+        }
+        ob[bf][b][jl] = sum16(o) * scale;   // the column's 16 lanes hold the same value
       }
-      o = (float2){sum16(o.x) * scale, sum16(o.y) * scale};
-      if (rg == 0) *(float2 *)&ob[b][jl] = o;
-    }
-    __syncthreads();                 // ob complete; the block's inputs read
-    {
-      const float2 o = *(const float2 *)&ob[tid >> 4][(tid & 15) * 2];
-      *(float2 *)(p.lin + (size_t)(b0 + (tid >> 4)) * p.ls + hv * DK + slice * WCOLS + (tid & 15) * 2) = o;
-    }
+    };
+    half(0);
+    // The other buffer's readers passed the last barrier; the next one shows
+    // it to every wave.
     if (more) land(bf ^ 1);
-    __syncthreads();
+    half(MAXB / 2);
+    lds_barrier();                   // ob complete, the next inputs in LDS
+    p.lin[(size_t)(b0 + (tid >> 5)) * p.ls + hv * DK + slice * WCOLS + (tid & 31)] = ob[bf][tid >> 5][tid & 31];
   }
   float *So = p.S_out + (size_t)hv * DK * DK;
 #pragma unroll
-  for (int r = 0; r < 8; ++r) *(float2 *)(So + (size_t)(i0 + r) * DK + j0) = s[r];
+  for (int r = 0; r < 8; ++r) So[(size_t)(i0 + r) * DK + j0] = s[r];
 }
 
 // Gated RMSNorm of the recurrence's outputs: one wave per (position, head).
@@ -553,7 +564,7 @@ int gdn_wide_launch(const cwen_gdn *g, float *lin, int ls, int zo, int ao, int b
   p.xc = xc; p.gates = gates; p.outh = outh; p.rflag = rflag;
   p.nkh = g->nkh; p.nvh = g->nvh; p.C = g->C; p.N = N;
   hipLaunchKernelGGL(gdn_wide_conv_kernel, dim3((unsigned)(g->C / DK + 1), (unsigned)((N + 15) / 16)), dim3(256), 0, st, p);
-  hipLaunchKernelGGL(gdn_wide_rec_kernel, dim3(DK / WCOLS, (unsigned)g->nvh), dim3(256), 0, st, p);
+  hipLaunchKernelGGL(gdn_wide_rec_kernel, dim3(DK / WCOLS, (unsigned)g->nvh), dim3(512), 0, st, p);
   hipLaunchKernelGGL(gdn_wide_norm_kernel, dim3((unsigned)g->nvh, (unsigned)((N + 3) / 4)), dim3(256), 0, st, p);
   CWEN_HIP_TRY(hipGetLastError());
   return CWEN_OK;
