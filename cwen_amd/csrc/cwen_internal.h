@@ -60,15 +60,16 @@ struct cwen_weight {
 
 // GatedDeltaNet layer state (gdn.hip): the recurrent state [nvh][dk][dk] in
 // two base slots, the conv history [C][3] in a ring of nslot slots, and the
-// pending inputs of the last block for a replay.  The device control word
+// pending inputs of the last block for a replay.  The control word
 // ctl[4] = {ring slot, base slot X, replay count L, pending parity P} is what
-// the kernels read; the host keeps a copy.
+// the kernels read; the host keeps a copy and, where it moves the state itself
+// (own_ctl), passes that by value outside graph captures.
 struct cwen_gdn {
   cwen_ctx *ctx;
   int nkh, nvh, dk, C;
   int nslot;
   int cur, X, L, P;         // host copy of ctl
-  int *ctl;                 // device control word
+  int *ctl;                 // control word: mapped host memory, or part of a model's device word
   int own_ctl;              // ctl allocated by this object (else part of a model's)
   int last_B;               // positions of the last, uncommitted block (0: none)
   float *S, *H;             // device: base states [2][nvh][dk][dk], history ring [nslot][C][3]

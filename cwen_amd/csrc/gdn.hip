@@ -54,14 +54,17 @@ constexpr int COLS = 16;            // columns of a head per recurrence workgrou
 
 __device__ __forceinline__ float silu_ref(float x) { return x * (1.f / (1.f + expf(-x))); }
 
-// Control word ctl[4] (device): ring slot, base slot X, replay count L,
-// pending parity P.  Block inputs go to pending buffer P; a replay reads
-// buffer P ^ 1 (the previous block's).
+// Control word: ring slot, base slot X, replay count L, pending parity P, read
+// from ctl, or with ctl null passed by value (a layer whose state the host
+// moves, outside graph capture: no read stands before the first loads).
+// Block inputs go to pending buffer P; a replay reads buffer P ^ 1 (the
+// previous block's).
 struct GdnParams {
   float *S_base;              // two base states [2][nvh][DK][DK]
   float *H_slots;             // conv history ring [nslot][C][3]
   size_t s_floats, h_floats;  // floats per state / history slot
-  const int *ctl;
+  const int *ctl;             // nullable
+  int cv[4];                  // the word when ctl is null
   int nslot;
   int force_L0;               // replay nothing (the previous block was not committed)
   float *S_peek;              // peek: replay peek_L positions of buffer peek_buf from base X into S_peek, no block
@@ -91,7 +94,7 @@ struct GdnParams {
 __global__ __launch_bounds__(256) void gdn_conv_kernel(GdnParams p) {
   const int c = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y;
   if (c >= p.C) return;           // whole waves (C is a multiple of 128)
-  const int cur = p.ctl[0], P = p.ctl[3];
+  const int cur = p.ctl ? p.ctl[0] : p.cv[0], P = p.ctl ? p.ctl[3] : p.cv[3];
   const float *H_in = p.H_slots + (size_t)cur * p.h_floats + (size_t)c * 3;
   const float4 w = *(const float4 *)(p.kw + (size_t)c * 4);
   // inputs at positions b-3, b-2, b-1, b (history slot entries 0..2 are the
@@ -129,8 +132,8 @@ __global__ __launch_bounds__(64 * RW) void gdn_rec_kernel(GdnParams p) {
   const int hv = blockIdx.x, slice = wave;
   const int hk = hv % p.nkh;
   const bool peek = p.S_peek != nullptr;
-  const int X = p.ctl[1], P = p.ctl[3];
-  const int L = peek ? p.peek_L : (p.force_L0 ? 0 : p.ctl[2]);
+  const int X = p.ctl ? p.ctl[1] : p.cv[1], P = p.ctl ? p.ctl[3] : p.cv[3];
+  const int L = peek ? p.peek_L : (p.force_L0 ? 0 : p.ctl ? p.ctl[2] : p.cv[2]);
   const int Pr = peek ? p.peek_buf : (P ^ 1);
   const int B = peek ? 0 : p.B;
   const int rg = lane & 15, cg = lane >> 4;
@@ -502,12 +505,13 @@ __global__ __launch_bounds__(256) void gdn_wide_norm_kernel(GdnWide p) {
 
 }  // namespace
 
-static void fill_params(GdnParams &p, const cwen_gdn *g) {
+static void fill_params(GdnParams &p, const cwen_gdn *g, bool by_value) {
   p.s_floats = (size_t)g->nvh * DK * DK;
   p.h_floats = (size_t)g->C * 3;
   p.S_base = g->S;
   p.H_slots = g->H;
-  p.ctl = g->ctl;
+  p.ctl = by_value ? nullptr : g->ctl;
+  p.cv[0] = g->cur; p.cv[1] = g->X; p.cv[2] = g->L; p.cv[3] = g->P;
   p.nslot = g->nslot;
   p.force_L0 = 0;
   p.S_peek = nullptr;
@@ -531,7 +535,14 @@ int gdn_block_launch(const cwen_gdn *g, const float *qkv, int qs, const float *z
                      float *out, int os, int B, hipStream_t st, _Float16 *outh, int ohs, const float *A,
                      const float *dt, int force_L0, int *rflag, bool conv_done) {
   GdnParams p;
-  fill_params(p, g);
+  bool by_value = g->own_ctl;
+  if (by_value) {
+    // A captured block must follow the layer's state when it is replayed.
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    CWEN_HIP_TRY(hipStreamIsCapturing(st, &cs));
+    by_value = cs == hipStreamCaptureStatusNone;
+  }
+  fill_params(p, g, by_value);
   p.force_L0 = force_L0;
   p.qkv = qkv; p.qs = qs;
   p.z = z; p.zs = zs;
@@ -572,7 +583,7 @@ int gdn_wide_launch(const cwen_gdn *g, float *lin, int ls, int zo, int ao, int b
 
 int gdn_peek_launch(const cwen_gdn *g, int L, int buf, float *S_out, hipStream_t st) {
   GdnParams p;
-  fill_params(p, g);
+  fill_params(p, g, g->own_ctl);
   p.S_peek = S_out;
   p.peek_L = L;
   p.peek_buf = buf;

@@ -796,7 +796,7 @@ int cwen_model_create(cwen_ctx *ctx, const cwen_model_cfg *cfg, cwen_model **out
     y.linear = !is_full(c, l);
     if (y.linear) {
       if (!(rc = cwen_gdn_create(ctx, c.gdn_nkh, c.gdn_nvh, 128, &y.gdn))) {
-        (void)hipFree(y.gdn->ctl);  // every layer's state moves with the model's commit
+        (void)hipHostFree(y.gdn->ctl);  // every layer's state moves with the model's commit
         y.gdn->ctl = m->ctl + 1;
         y.gdn->own_ctl = 0;
         rc = gemv_alloc_q4(ctx, H, R.lin, &y.lin_in);

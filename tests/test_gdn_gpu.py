@@ -179,3 +179,35 @@ def test_gdn_argument_errors(env):
     with pytest.raises(gpu.CwenError):
         G.get_state(1)
     G.free()
+
+
+@pytest.mark.parametrize("keep", [8, 0])
+def test_captured_block_follows_the_state(env, keep):
+    """Blocks launched directly get the layer's control word by value, captured
+    ones read it: every replay of one captured block equals the eager block from
+    the same state, across commits made between the replays (of the whole block
+    or none of it: a replayed prefix is applied once, and here each block runs twice)."""
+    torch, gpu, ctx = env
+    nkh, nvh, B = 2, 4, 8
+    S, hist, kw, wn, qkv, z, decay, beta = _inputs(31, B, nkh, nvh)
+    dev = [torch.from_numpy(a).cuda() for a in (qkv, z, decay, beta, kw, wn)]
+    out = [torch.zeros(B, nvh * 128, device="cuda") for _ in range(2)]
+    layers = [gpu.GDN(ctx, nkh, nvh) for _ in range(2)]
+    for g in layers:
+        g.set_state(S, hist)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        layers[1].block(*dev, out[1], B, stream=side)
+    for i in range(4):
+        print("captured block, replay", i, flush=True)
+        layers[0].block(*dev, out[0], B)
+        if i:   # the host's record that a block is outstanding; its launch starts from the same state
+            layers[1].block(*dev, out[1], B)
+            torch.cuda.synchronize()
+            out[1].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[0], out[1]), i
+        for g in layers:
+            g.commit(keep)
