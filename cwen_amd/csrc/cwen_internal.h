@@ -322,13 +322,19 @@ int gdn_wide_launch(const cwen_gdn *g, float *lin, int ls, int zo, int ao, int b
 int gdn_peek_launch(const cwen_gdn *g, int L, int buf, float *S_out, hipStream_t st);
 
 // ------------------------------------------------------------ model.hip
+// Tokens of a block by value (out not null): the embedding reads them from its
+// arguments and leaves them in out[0 .. B-1] for the launches after it.
+struct EmbedToks {
+  int *out;
+  int t[CWEN_BMAX];
+};
 // Also writes each row's sum of squares to ssq[b][0] (one partial per column)
 // and, when xh is given, the f16 operand x * nw of the first RMSNorm (row-major, or
 // with `tiled` in wide_at's order).
 // rflag (nullable) is set to 1 when an f16 value written is not finite.
 int embed_launch(const uint8_t *qs, const uint16_t *sc, int type, const int *toks, int B, int H, float *X,
                  int xs, float *ssq, hipStream_t st, _Float16 *xh = nullptr, const float *nw = nullptr,
-                 int *rflag = nullptr, bool tiled = false);
+                 int *rflag = nullptr, bool tiled = false, const EmbedToks *tv = nullptr);
 size_t attn_partial_floats(int NH, int NKV, int max_ctx, int B);
 int attention_init();
 // Largest query heads per KV head the attention kernels take at every block

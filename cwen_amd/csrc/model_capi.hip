@@ -76,7 +76,7 @@ struct cwen_model {
   _Float16 *yh = nullptr;        // attention output f16 [BMAX][NH*HD]
   _Float16 *hh = nullptr;        // FFN hidden f16 [BMAX][I]
   float *logits = nullptr;       // [BMAX][V]
-  int *hres = nullptr;           // pinned host copy of res
+  int *hres = nullptr;           // res in mapped host memory, written by the block's last launch
   // Workspace of cwen_model_prefill for `wn` positions at a time (0: not
   // allocated), the block scratch above at that length.
   int wn = 0;
@@ -174,10 +174,18 @@ int upload_w(cwen_model *m, int type, const void *data, const void *scales, int 
 // Device commit of a block of nmax positions: keep n, or walk[0] + 1
 // (accepted drafts + bonus) when walk is given, clamped to [1, nmax].  The
 // position and the GDN ring slot advance by n; the GDN base state and replay
-// count follow gdn_commit_host's rule.  The sticky range flag ctl[5] is
-// copied to *flag_out, next to the walk's result, for the host to read.
-__global__ void advance_kernel(int *ctl, const int *walk, int n, int nmax, int nslot, int *flag_out) {
-  *flag_out = ctl[5];
+// count follow gdn_commit_host's rule.  The sticky range flag ctl[5] goes to
+// res[0], next to the walk's result.
+// It is also the block's last launch, so it hands the result words to the host
+// (hres, mapped host memory, nullable): with a copy after it, and one for the
+// tokens before the first launch, a serial step took about 9 us longer.
+__global__ void advance_kernel(int *ctl, const int *walk, int n, int nmax, int nslot, int *res, int *hres) {
+  const int i = threadIdx.x;
+  if (hres && i > 0 && i < 3 + CWEN_BMAX) hres[i] = res[i];
+  if (i > 0) return;
+  const int flag = ctl[5];
+  res[0] = flag;
+  if (hres) hres[0] = flag;
   if (walk) n = walk[0] + 1;
   n = n < 1 ? 1 : (n > nmax ? nmax : n);
   ctl[0] += n;
@@ -341,7 +349,7 @@ int mtp_commit_pass(cwen_model *m, int B, int mode, hipStream_t st) {
   return CWEN_OK;
 }
 
-int block(cwen_model *m, int B, int mode, hipStream_t st) {
+int block(cwen_model *m, int B, int mode, hipStream_t st, const int *toks = nullptr) {
   const cwen_model_cfg &c = m->cfg;
   cwen_ctx *ctx = m->ctx;
   const int H = c.d_model, I = c.d_ffn;
@@ -355,8 +363,10 @@ int block(cwen_model *m, int B, int mode, hipStream_t st) {
   // Every f16 operand written raises the sticky flag ctl[5] when it is out
   // of f16's range.
   int *const rflag = m->ctl + 5;
+  EmbedToks tv = {m->toks, {}};
+  if (toks) memcpy(tv.t, toks, (size_t)B * sizeof(int));
   if ((rc = embed_launch(m->emb_qs, m->emb_sc, m->emb_type, m->toks, B, H, m->X, H, m->ssq, st, m->xh,
-                         m->L[0].attn_norm, rflag)))
+                         m->L[0].attn_norm, rflag, false, toks ? &tv : nullptr)))
     return rc;
   int npart = 1;
   for (int l = 0; l < c.n_layers; ++l) {
@@ -419,8 +429,8 @@ int block(cwen_model *m, int B, int mode, hipStream_t st) {
     if ((rc = gemv_launch(ctx, m->head, 1, 0, GEMV_EPI_ARGMAX, m->xh, o, B, st, nullptr, &nh))) return rc;
   }
   if (mtp_ready(m) && (rc = mtp_commit_pass(m, B, mode, st))) return rc;
-  hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(1), 0, st, m->ctl, mode == MODE_VERIFY ? m->res + 1 : nullptr, B,
-                     B, CWEN_BMAX + 1, m->res);
+  hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(64), 0, st, m->ctl, mode == MODE_VERIFY ? m->res + 1 : nullptr, B,
+                     B, CWEN_BMAX + 1, m->res, mode != MODE_FWD ? m->hres : nullptr);
   CWEN_HIP_TRY(hipGetLastError());
   return CWEN_OK;
 }
@@ -559,17 +569,17 @@ void drop_graphs(cwen_model *m) {
         }
 }
 
-// Stage the tokens, then run the block: replay its graph (captured on first
-// use) or launch eagerly.
+// Run the block: launch eagerly, the tokens by value, or stage the tokens and
+// replay its graph (captured on first use).
 int run_block(cwen_model *m, const int *toks, int B, int mode, hipStream_t st) {
   for (int b = 0; b < B; ++b)
     if (toks[b] < 0 || toks[b] >= m->cfg.vocab) return CWEN_EINVAL;
+  // the MTP commit's launch shape depends on the position: eager
+  if (!m->use_graphs || mtp_ready(m)) return block(m, B, mode, st, toks);
   CWEN_HIP_TRY(hipEventSynchronize(m->tok_ev));  // the previous staging copy has been read
   memcpy(m->htok, toks, (size_t)B * sizeof(int));
   CWEN_HIP_TRY(hipMemcpyAsync(m->toks, m->htok, (size_t)B * sizeof(int), hipMemcpyHostToDevice, st));
   CWEN_HIP_TRY(hipEventRecord(m->tok_ev, st));
-  // the MTP commit's launch shape depends on the position: eager
-  if (!m->use_graphs || mtp_ready(m)) return block(m, B, mode, st);
   hipGraphExec_t &ge = m->gexec[mode][attention_wide(m->pos + B)][B - 1];
   if (!ge) {
     hipGraph_t g = nullptr;
@@ -1050,7 +1060,6 @@ int cwen_model_forward(cwen_model *m, const int *toks, int B, int want_argmax, i
   int rc;
   if ((rc = run_block(m, toks, B, want_argmax ? MODE_FWD_HEAD : MODE_FWD, st))) return rc;
   if (want_argmax) {
-    CWEN_HIP_TRY(hipMemcpyAsync(m->hres, m->res, (3 + B) * sizeof(int), hipMemcpyDeviceToHost, st));
     CWEN_HIP_TRY(hipStreamSynchronize(st));
     if (argmax_out) memcpy(argmax_out, m->hres + 3, (size_t)B * sizeof(int));
   }
@@ -1096,7 +1105,6 @@ int cwen_model_verify(cwen_model *m, const int *blk, int B, int *k_out, int *bon
   hipStream_t st = (hipStream_t)stream;
   int rc;
   if ((rc = run_block(m, blk, B, MODE_VERIFY, st))) return rc;
-  CWEN_HIP_TRY(hipMemcpyAsync(m->hres, m->res, 3 * sizeof(int), hipMemcpyDeviceToHost, st));
   CWEN_HIP_TRY(hipStreamSynchronize(st));
   const int k = m->hres[1];
   if (k < 0 || k > B - 1) return CWEN_EHIP;
