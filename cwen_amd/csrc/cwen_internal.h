@@ -40,9 +40,12 @@ struct cwen_ctx {
 // A GEMV launch's work decomposition (gemv.hip): grid workgroups, the first
 // nsplit of which take pieces (S per tile, rps rounds each) of row tiles
 // tile0 .. tile0 + nsplit / S - 1; the others take whole row tiles.
+// kw: the K split of every row inside one workgroup instead (gemv_kw.hip; S
+// pieces of rps rounds, all tiles counted as split).
 struct GemvGrid {
-  int grid, nsplit, S, rps, tile0;
+  int grid, nsplit, S, rps, tile0, kw;
 };
+constexpr int GEMV_KW_MAX = 6;
 
 struct cwen_weight {
   cwen_ctx *ctx;
@@ -54,7 +57,7 @@ struct cwen_weight {
   uint8_t *dev;             // tiled device data
   size_t bytes;             // device bytes of the tiled data
   size_t src_bytes;         // bytes of the reference layout (qs + scales)
-  GemvGrid cfg[2];          // decomposition for one side / both sides of a pair (shape-only)
+  GemvGrid cfg[2];          // decomposition for one side / both sides of a pair (shape-only); PAIR: see gemv_launch
   int rows;                 // row groups per wave (shape-only)
 };
 
@@ -161,6 +164,13 @@ __device__ __forceinline__ void lds_barrier() {
 // run.c:378-384 silu_one: x * (1 / (1 + exp(-x)))
 __device__ __forceinline__ float silu_f(float x) { return x * (1.f / (1.f + expf(-x))); }
 
+// The 4-tap conv of one channel (run.c:2183-2200) at inputs a..d = positions
+// b-3 .. b, w the taps.  Written as FMAs: left as products and sums, the
+// compiler contracts them, and not the same way in every kernel.
+__device__ __forceinline__ float conv4(float a, float b, float c, float d, float4 w) {
+  return fmaf(d, w.w, fmaf(c, w.z, fmaf(a, w.x, b * w.y)));
+}
+
 // An f16 operand that is not finite: the f32 value left f16's range (or was
 // not finite itself).  Writers of f16 operands raise a sticky flag, which the
 // model's entry points report.
@@ -190,8 +200,8 @@ __device__ __forceinline__ _Float16 f16_mul(float a, float b) {
 // 2 of an L2's 16 channels.
 __device__ __forceinline__ size_t wide_at(int c, int k, int N) { return ((size_t)(k >> 7) * N + c) * 128 + (k & 127); }
 
-// Row-tile partials of a column's sum of squares: at most 128 per column.
-constexpr int CWEN_MAX_PARTS = 128;
+// Partials of a column's sum of squares, one per 16 rows: at most 512.
+constexpr int CWEN_MAX_PARTS = 512;
 
 // ------------------------------------------------------------ gemv.hip
 enum { GEMV_EPI_STORE = 0, GEMV_EPI_PAIR = 1, GEMV_EPI_SWIGLU = 2, GEMV_EPI_ARGMAX = 3, GEMV_EPI_CONV = 4 };
@@ -209,7 +219,7 @@ struct GemvOut {
   int ys;
   int accumulate;    // y += result
   ArgmaxOut am;      // ARGMAX only
-  float *ssq;        // STORE: per row tile, the sum of squares of the final y per column [CWEN_BMAX][CWEN_MAX_PARTS]
+  float *ssq;        // STORE: per 16 rows, the sum of squares of the final y per column [CWEN_BMAX][CWEN_MAX_PARTS]
   const float *nwh;  // with yh: the f16 copy holds y * nwh[row] (the next RMSNorm's weight), nullable
   // CONV (a STORE whose rows < cv_C are GatedDeltaNet q/k/v channels): they get the
   // depthwise causal conv + SiLU (run.c conv1d_update) instead of a store:
@@ -259,8 +269,11 @@ struct GemvScratch {
 };
 // Whether a decomposition's split pieces fit the given scratch.
 bool gemv_grid_fits(const GemvGrid &g, size_t partials_floats, int ncounters);
-// Row tiles of a launch over w: the number of ssq partials it writes.
-int gemv_row_tiles(const cwen_weight *w);
+// Number of ssq partials a launch over w writes per column.
+int gemv_ssq_parts(const cwen_weight *w);
+// gemv_kw.hip: params is gemv.hip's GemvParams.
+int gemv_kw_init();   // once per device, before the first launch
+int gemv_kw_launch(int fmt, int epi, const void *params, hipStream_t st);
 // post (f16 operand only): the operand is w * x with x not yet normalised;
 // each output column c is scaled by 1 / sqrt(sum_p post->ssq[c][p] / K +
 // post->eps), completing the RMSNorm (post->x, post->w unused).
@@ -282,7 +295,7 @@ struct WideOut {
   int accumulate;    // y += result
   _Float16 *yh;      // SWIGLU: silu(A)*B; STORE (nullable): y * nwh[row]; in wide_at's order
   const float *nwh;
-  float *ssq;        // STORE, nullable: sums of squares of y per 64 rows [c][CWEN_MAX_PARTS]
+  float *ssq;        // STORE, nullable: sums of squares of y per 16 rows [c][CWEN_MAX_PARTS]
   int *rflag;        // set to 1 when an f16 value written is not finite
 };
 // Whether wide_gemm takes the weight (finish: as an accumulating STORE, whose

@@ -105,9 +105,7 @@ __global__ __launch_bounds__(256) void gdn_conv_kernel(GdnParams p) {
     const int t = b - 3 + j;
     in[j] = t >= 0 ? p.qkv[(size_t)t * p.qs + c] : H_in[t + 3];
   }
-  // ((st0*w0 + st1*w1) + st2*w2) + xin*w3, each product and sum rounded
-  const float x = __fadd_rn(__fadd_rn(__fadd_rn(__fmul_rn(in[0], w.x), __fmul_rn(in[1], w.y)), __fmul_rn(in[2], w.z)),
-                            __fmul_rn(in[3], w.w));
+  const float x = conv4(in[0], in[1], in[2], in[3], w);
   float y = silu_ref(x);
   float *hs = p.H_slots + (size_t)((cur + 1 + b) % p.nslot) * p.h_floats + (size_t)c * 3;
   hs[0] = in[1]; hs[1] = in[2]; hs[2] = in[3];
@@ -362,9 +360,7 @@ __global__ __launch_bounds__(256) void gdn_wide_conv_kernel(GdnWide p) {
     float y[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      const float x = __fadd_rn(__fadd_rn(__fadd_rn(__fmul_rn(in[e][k], w[k].x), __fmul_rn(in[e + 1][k], w[k].y)),
-                                          __fmul_rn(in[e + 2][k], w[k].z)),
-                                __fmul_rn(in[e + 3][k], w[k].w));
+      const float x = conv4(in[e][k], in[e + 1][k], in[e + 2][k], in[e + 3][k], w[k]);
       y[k] = silu_ref(x);
     }
     if (h < 2 * p.nkh) {

@@ -63,9 +63,6 @@
 
 namespace {
 
-constexpr int TILES = Q4_ST_TILES;  // tiles per round: one super-tile per stream
-// A per-lane buffer offset past any activation range: the load returns zeros.
-constexpr uint32_t kPastRange = 0xFFFFFFE0u;
 constexpr int WAVES = 4;            // waves per workgroup
 
 // K-run order inside a dword: the nibble unpack yields elements from nibbles
@@ -122,40 +119,6 @@ __device__ void argmax_finish(const unsigned long long *key, int B, const Argmax
   }
 }
 
-struct GemvParams {
-  const uint8_t *w;    // super-tiled weights, round-major: super-tile (st, rg, side) at ((st*nrg + rg)*nsw + side)
-  uint32_t wbytes;     // bytes of the tiled weights (buffer range)
-  int nsw;             // sides stored per super-tile position (1 or 2)
-  int side0;           // first side computed (NS == 1)
-  int M, nrg, nst;
-  // Workgroups [0, nsplit) each take one piece of a split row tile: piece
-  // i % S (rounds (i % S) * rps ..) of tile tile0 + i / S.  The others take
-  // whole row tiles 0, 1, ...
-  int nsplit, S, rps, tile0;
-  const _Float16 *xh;  // activations f16 [B][K]
-  uint32_t xbytes;     // buffer range of the activations: columns >= B read as zero
-  const float *xf;     // XN: f32 rows [c*xfs + k], converted to f16 while staging
-  int xfs;
-  // Post-scale (f16 operand w * x, x not yet normalised): output column c is
-  // multiplied by 1 / sqrt(sum_p pss[p][c] / K + eps).
-  const float *pss;
-  int pnpart;
-  float eps;
-  int K, B;
-  float *part;         // split-K partials
-  int *cnt;            // per split-tile arrival counters (zero between launches)
-  GemvOut out;
-};
-
-// 8 f32 activations -> 8 f16, rounded to nearest.
-__device__ __forceinline__ uint4 cvt8(const uint4 (&x)[2]) {
-  const float4 x0 = __builtin_bit_cast(float4, x[0]), x1 = __builtin_bit_cast(float4, x[1]);
-  const half2_t h0 = {(_Float16)x0.x, (_Float16)x0.y}, h1 = {(_Float16)x0.z, (_Float16)x0.w};
-  const half2_t h2 = {(_Float16)x1.x, (_Float16)x1.y}, h3 = {(_Float16)x1.z, (_Float16)x1.w};
-  return make_uint4(__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1),
-                    __builtin_bit_cast(uint32_t, h2), __builtin_bit_cast(uint32_t, h3));
-}
-
 // FMT: weight format.  NS: sides of an interleaved pair computed (2: both;
 // the two waves of a wave pair take sides 0 and 1 of the same row group and
 // combine them through LDS).  EPI: epilogue.  CB: activation columns staged
@@ -175,6 +138,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
   // the same LDS for its exchanges, so a workgroup holds CB * 2 KB.
   __shared__ uint4 act[2][CB * 64];          // [buf][column c][unit u ^ c], f16 x 8 per unit
   __shared__ int s_last;
+  __shared__ float s_psc[CWEN_BMAX];
 
   const int tid = threadIdx.x;
   // Wave index as a scalar: loop bounds and addresses are then provably
@@ -191,17 +155,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
   const int st0 = sp * p.rps;
   const int nround = split ? min(p.nst - st0, p.rps) : p.nst;
 
-  // Post-scale: the producer's partial sums of squares of every staged
-  // column, loaded first, so that waiting for them waits for nothing else
-  // (see psc below).  ssq is [column][CWEN_MAX_PARTS = 128], so a wave's
-  // load of 64 partials of one column is one contiguous 256-byte run, and the
-  // loads need no guard.
-  float pp[2][CB];
+  // Post-scale: the producer's partial sums of squares, wave w those of
+  // columns w, w + 4, ..., loaded first, so that waiting for them waits for
+  // nothing else.
+  PostParts pp[CB / WAVES];
   if (p.pss) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int c = 0; c < CB; ++c) pp[j][c] = p.pss[c * CWEN_MAX_PARTS + lane + 64 * j];
+    for (int c = 0; c < CB / WAVES; ++c) post_load(pp[c], p.pss + (wave + WAVES * c) * CWEN_MAX_PARTS, p.pnpart, lane);
   }
   __builtin_amdgcn_sched_barrier(0);
   const __amdgpu_buffer_rsrc_t wr = make_rsrc(p.w, p.wbytes);
@@ -288,23 +248,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
       __builtin_amdgcn_sched_barrier(0);  // issue the ring in slot order
     }
   }
-  // Post-scale: the scales of this lane's output columns 4g .. 4g+3, while
-  // the first round's weights are in flight.  Lane p adds partials p and
-  // p + 64 in that order, then one DPP tree over the wave: a
-  // fixed order, so every workgroup and every block size gets the same scale
-  // for a column.  Every column index is a compile-time constant and nothing
-  // branches per column (a private array indexed at run time would move to
-  // LDS; a uniform branch per column reloads kernel arguments).
-  float psc[4] = {1.f, 1.f, 1.f, 1.f};
+  // Their scales, while the first round's weights are in flight; every wave
+  // reads those of its outputs from LDS in the epilogue, barriers later.
   if (p.pss) {
-    const float kf = (float)p.K, eps = p.eps;
-    const int nb = p.B, np = p.pnpart;
 #pragma unroll
-    for (int c = 0; c < CB; ++c) {
-      float v = lane < np ? pp[0][c] : 0.f;
-      if (lane + 64 < np) v += pp[1][c];
-      const float sc1 = 1.f / sqrtf(sum64(v) / kf + eps);
-      psc[c & 3] = ((c >> 2) == g && c < nb) ? sc1 : psc[c & 3];
+    for (int c = 0; c < CB / WAVES; ++c) {
+      const float sc1 = post_scale(pp[c], (float)p.K, p.eps);
+      if (lane == 0) s_psc[wave + WAVES * c] = sc1;
     }
   }
   auto stage_store = [&](uint4 *buf) __attribute__((always_inline)) {
@@ -511,7 +461,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
 
   if (p.pss) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) res[e] *= psc[e];
+    for (int e = 0; e < 4; ++e) res[e] *= s_psc[(g * 4 + e) & (CB - 1)];   // columns past CB are discarded
   }
   const GemvOut &o = p.out;
   const int row = rg * Q4_ROWS + n;
@@ -568,36 +518,8 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
   float sq[4] = {0.f, 0.f, 0.f, 0.f};  // this lane's share of the row tile's sum of squares
   bool bad = false;                    // an f16 copy out of range
   if constexpr (NS == 1 && EPI == GEMV_EPI_CONV) {
-    // GatedDeltaNet conv rows: lane (g, n) holds positions 4g .. 4g+3 of
-    // channel `row`; positions 4g-3 .. 4g-1 come from lane (g-1, n), or for
-    // g = 0 from the history slot the block starts from.
     if (cv_rows) {
-      const float p1 = __shfl(res[1], lane - 16), p2 = __shfl(res[2], lane - 16), p3 = __shfl(res[3], lane - 16);
-      if (store) {
-        const int cur = cv_cur, P = cv_P;
-        const size_t hf = (size_t)o.cv_C * 3;
-        float a[7];
-        a[0] = g == 0 ? cv_h[0] : p1;
-        a[1] = g == 0 ? cv_h[1] : p2;
-        a[2] = g == 0 ? cv_h[2] : p3;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) a[3 + e] = res[e];
-        const float4 w = cv_w4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int b = g * 4 + e;
-          if (b >= p.B) continue;
-          // ((st0*w0 + st1*w1) + st2*w2) + xin*w3, each product and sum rounded
-          const float x = __fadd_rn(__fadd_rn(__fadd_rn(__fmul_rn(a[e], w.x), __fmul_rn(a[e + 1], w.y)),
-                                              __fmul_rn(a[e + 2], w.z)),
-                                    __fmul_rn(a[e + 3], w.w));
-          o.cv_xc[((size_t)P * CWEN_BMAX + b) * o.cv_C + row] = silu_f(x);
-          float *hs = o.cv_H + (size_t)((cur + 1 + b) % o.cv_nslot) * hf + (size_t)row * 3;
-          hs[0] = a[e + 1];
-          hs[1] = a[e + 2];
-          hs[2] = a[e + 3];
-        }
-      }
+      conv_store(o, res, cv_h, cv_w4, cv_cur, cv_P, row, lane, g, p.B, store);
       store = false;
     }
   }
@@ -634,23 +556,12 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
   }
   if (bad) raise_flag(o.rflag);
   if (o.ssq) {
-    // Sum of squares of this row tile's outputs per column, in a fixed order
-    // (rows of a wave by the DPP tree, then row groups in order): ssq[c][rt],
-    // the partials a normalising consumer sums.  (STORE only: NS == 1, so
-    // slot == ws.)
-    float *const s_sq = (float *)&act[0][0];   // [SPW][16]
+    // Sum of squares of this row group's outputs per column, the partials a
+    // normalising consumer sums.  (STORE only: NS == 1.)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) sq[e] = sum16(sq[e]);
-    if (carry && n == 0) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s_sq[ws * 16 + g * 4 + e] = sq[e];
-    }
-    __syncthreads();
-    if (tid < 16 && tid < p.B) {
-      float t = s_sq[tid];
-#pragma unroll
-      for (int w = 1; w < SPW; ++w) t += s_sq[w * 16 + tid];
-      o.ssq[tid * CWEN_MAX_PARTS + rt] = t;
+    for (int e = 0; e < 4; ++e) {
+      sq[e] = sum16(sq[e]);
+      if (n == 0 && rg < p.nrg && g * 4 + e < p.B) o.ssq[(g * 4 + e) * CWEN_MAX_PARTS + rg] = sq[e];
     }
   }
 }
@@ -1009,7 +920,7 @@ int gemv_repack_part(cwen_weight *w, const uint8_t *dsrc, const uint16_t *dsc, i
 // at most (one 16-row stream per wave) and one arrival counter per split
 // tile.
 bool gemv_grid_fits(const GemvGrid &g, size_t partials_floats, int ncounters) {
-  return g.nsplit == 0 || ((size_t)g.nsplit * WAVES * 256 <= partials_floats && g.nsplit / g.S <= ncounters);
+  return g.kw || g.nsplit == 0 || ((size_t)g.nsplit * WAVES * 256 <= partials_floats && g.nsplit / g.S <= ncounters);
 }
 
 namespace {
@@ -1058,17 +969,39 @@ double grid_cost(int ncu, int nst, const GemvGrid &c, double extra) {
   return worst + extra;
 }
 
-// Decomposition of ntile row tiles of nst rounds.  A launch with fewer tiles
-// than CUs splits every tile into S pieces (at least two rounds each)
-// for at most wg_per_cu workgroups per CU.  A larger one takes whole tiles,
+// Decomposition of ntile row tiles (nrg row groups) of nst rounds.
+// Small weights (kw): K split over the waves of a workgroup per row group, for
+// about 7 waves per CU, when tiles are at most half as many as CUs, a wave gets
+// at most 3 rounds and the weight has at most 18 MB.  With more row groups than
+// CUs, some of which then run two workgroups, at most 2 rounds and, unless Q4_0, 14
+// MB: 4300 x 7680 (269 groups, 3 rounds) 8.9-11.9 against 9.0-10.3, Q4_1 5120 x 5120
+// f32 at B = 4 9.1 against 8.2 us.  Measured against the forms below, f16 in, B = 1 / 4 /
+// 8 / 16: 5120 x 6144 (3840 super-tiles, 2 rounds) 7.3 / 8.3 / 8.9 / 9.3 against 8.6 / 8.8 / 8.9
+// / 9.4 us, 2048 x 6144 5.1 / 5.8 / 6.1 / 6.9 against 7.4 / 7.6 / 7.7 / 8.0,
+// 1000 x 2080 4.5 / 4.5 / 4.6 / 4.8 against 6.6 / 7.1 / 7.1 / 7.5.  Past it a wave's own
+// activation staging shows: 5120 x 17408 (6 rounds) 15.6 / 17.2 / 19.7 / 26.6
+// against 13.8 / 14.1 / 14.7 / 15.6, Q5_K 5120 x 6144 (23.6 MB) 9.2 / 9.9 / 10.5 /
+// 11.1 against 9.3 / 9.5 / 9.7 / 10.2, 64 x 17408, 4 workgroups, 8.6 against 7.6, and with
+// more tiles 10240 x 2048 at B = 16 8.5 against 6.6.
+// Otherwise a launch with fewer tiles than CUs splits every tile into S pieces
+// (at least two rounds each) for at most wg_per_cu workgroups per CU.  A larger one takes whole tiles,
 // except that the ntile mod ncu remainder tiles are split into the pieces
 // (chosen by grid_cost) that spread them over the CUs: without that, the
 // CUs that get one whole tile more than the others would set the launch's
 // length.
 // split_basis: the tile count that sizes the split (the single-side one for
-// both launch kinds, so a pair launch splits K as its single sides do).
-GemvGrid choose_grid(const cwen_ctx *ctx, int ntile, int nst, int split_basis) {
-  GemvGrid best = {ntile, 0, 1, nst, 0};
+// both launch kinds, so a pair launch splits K as its single sides do); bytes:
+// of one side; kw: allowed (a SwiGLU launch puts both sides into one workgroup: at 352
+// row groups x 4 rounds, B = 16, 9.0 us against 8.0 in whole tiles).
+GemvGrid choose_grid(const cwen_ctx *ctx, int ntile, int nst, int split_basis, int nrg, size_t bytes, int fmt, bool kw) {
+  GemvGrid best = {ntile, 0, 1, nst, 0, 0};
+  if (kw && 2 * split_basis <= ctx->ncu && bytes <= (size_t)18 << 20) {
+    const int S0 = std::min({std::max(7 * ctx->ncu / nrg, 1), GEMV_KW_MAX, nst});
+    const int rps = (nst + S0 - 1) / S0, S = (nst + rps - 1) / rps;
+    const bool one_wave_of_groups = nrg <= ctx->ncu;
+    if (one_wave_of_groups ? rps <= 3 : rps <= 2 && (fmt == GEMV_Q4 || bytes <= (size_t)14 << 20))
+      return {ntile * S, ntile * S, S, rps, 0, 1};
+  }
   // More than half as many tiles as CUs: whole tiles, one per CU.  Split in
   // two, most CUs would get two pieces of the same total length plus the
   // partials' round trip (measured at 224 tiles of 10 rounds: 10.7 us whole,
@@ -1082,7 +1015,7 @@ GemvGrid choose_grid(const cwen_ctx *ctx, int ntile, int nst, int split_basis) {
     int S = std::min(std::max(target / split_basis, 1), std::max(nst / 2, 1));
     const int rps = (nst + S - 1) / S;
     S = (nst + rps - 1) / rps;
-    const GemvGrid cand = {ntile * S, ntile * S, S, rps, 0};
+    const GemvGrid cand = {ntile * S, ntile * S, S, rps, 0, 0};
     if (S > 1 && gemv_grid_fits(cand, ctx->partials_floats, ctx->ncounters)) best = cand;
     return best;
   }
@@ -1091,7 +1024,7 @@ GemvGrid choose_grid(const cwen_ctx *ctx, int ntile, int nst, int split_basis) {
   double best_cost = grid_cost(ctx->ncu, nst, best, 0.0);
   for (int s = 2; s <= nst / 2; ++s) {
     const int r = (nst + s - 1) / s, se = (nst + r - 1) / r;
-    const GemvGrid part = {rem * se + ntile - rem, rem * se, se, r, ntile - rem};
+    const GemvGrid part = {rem * se + ntile - rem, rem * se, se, r, ntile - rem, 0};
     if (se != s || !gemv_grid_fits(part, ctx->partials_floats, ctx->ncounters)) continue;
     const double c = grid_cost(ctx->ncu, nst, part, kSplitEarly);
     if (c < best_cost) {
@@ -1111,11 +1044,12 @@ void gemv_choose_split(const cwen_ctx *ctx, cwen_weight *w) {
   const int single = (w->nrg + tile_rows(1) - 1) / tile_rows(1);
   for (int ns = 1; ns <= w->nside; ++ns) {
     const int rpw = tile_rows(ns);
-    w->cfg[ns - 1] = choose_grid(ctx, (w->nrg + rpw - 1) / rpw, w->nst, single);
+    w->cfg[ns - 1] = choose_grid(ctx, (w->nrg + rpw - 1) / rpw, w->nst, single, w->nrg, w->bytes / w->nside, w->fmt,
+                                 ns == 1 || w->nrg <= ctx->ncu);
   }
 }
 
-int gemv_row_tiles(const cwen_weight *w) { return (w->nrg + WAVES - 1) / WAVES; }
+int gemv_ssq_parts(const cwen_weight *w) { return w->nrg; }
 
 int gemv_launch(cwen_ctx *ctx, const cwen_weight *w, int nsides, int side0, int epi,
                 const _Float16 *xh, const GemvOut &out, int B, hipStream_t st, const GemvF32 *xf,
@@ -1123,7 +1057,7 @@ int gemv_launch(cwen_ctx *ctx, const cwen_weight *w, int nsides, int side0, int 
   if (post && (xf || !xh || !post->ssq || post->npart < 1 || post->npart > CWEN_MAX_PARTS)) return CWEN_EINVAL;
   if (xf && (xh || !xf->x || ((uintptr_t)xf->x & 15) || (xf->xs & 3) || (B > 1 && xf->xs < w->ne0)))
     return CWEN_EINVAL;
-  if (out.ssq && (epi != GEMV_EPI_STORE || gemv_row_tiles(w) > CWEN_MAX_PARTS)) return CWEN_EINVAL;
+  if (out.ssq && (epi != GEMV_EPI_STORE || gemv_ssq_parts(w) > CWEN_MAX_PARTS)) return CWEN_EINVAL;
   GemvParams p;
   p.w = w->dev;
   p.wbytes = (uint32_t)w->bytes;
@@ -1132,7 +1066,8 @@ int gemv_launch(cwen_ctx *ctx, const cwen_weight *w, int nsides, int side0, int 
   p.M = w->ne1;
   p.nrg = w->nrg;
   p.nst = w->nst;
-  GemvGrid cfg = w->cfg[nsides - 1];
+  // A pair's two sides with K split inside workgroups are launched side by side.
+  GemvGrid cfg = w->cfg[epi == GEMV_EPI_PAIR && w->cfg[0].kw ? 0 : nsides - 1];
   p.xh = xh;
   const int xfs = xf ? (B > 1 ? xf->xs : w->ne0) : 0;
   p.xbytes = xf ? (uint32_t)(((size_t)(B - 1) * xfs + w->ne0) * 4) : (uint32_t)((size_t)B * w->ne0 * 2);
@@ -1144,17 +1079,22 @@ int gemv_launch(cwen_ctx *ctx, const cwen_weight *w, int nsides, int side0, int 
   p.K = w->ne0;
   p.B = B;
   p.part = scr ? scr->partials : ctx->partials;
+  p.ncu = ctx->ncu;
   p.cnt = scr ? scr->counters : ctx->counters;
   p.out = out;
   const int rpw = tile_rows(nsides);
   const int ntile = (w->nrg + rpw - 1) / rpw;
-  if (epi == GEMV_EPI_ARGMAX) cfg = {ntile, 0, 1, w->nst, 0};  // final row values in one workgroup
+  if (epi == GEMV_EPI_ARGMAX) cfg = {ntile, 0, 1, w->nst, 0, 0};  // final row values in one workgroup
   if (scr && !gemv_grid_fits(cfg, scr->partials_floats, scr->ncounters)) return CWEN_ESCRATCH;
   p.nsplit = cfg.nsplit;
   p.S = cfg.S;
   p.rps = cfg.rps;
   p.tile0 = cfg.tile0;
   const int nrt = cfg.grid;
+  if (epi == GEMV_EPI_CONV && (!out.cv_w || !out.cv_H || !out.cv_xc || !out.cv_ctl || out.cv_C < 0 || out.cv_C > w->ne1 ||
+                               out.cv_C % Q4_ROWS || out.cv_nslot < 1))
+    return CWEN_EINVAL;
+  if (cfg.kw) return nsides == (epi == GEMV_EPI_SWIGLU || epi == GEMV_EPI_PAIR ? 2 : 1) ? gemv_kw_launch(w->fmt, epi, &p, st) : CWEN_EINVAL;
   int rc = CWEN_EINVAL;
   if (w->fmt == GEMV_Q4) {
     if (nsides == 2 && epi == GEMV_EPI_PAIR) {
@@ -1164,9 +1104,6 @@ int gemv_launch(cwen_ctx *ctx, const cwen_weight *w, int nsides, int side0, int 
       launch_cb<GEMV_Q4, 2, GEMV_EPI_SWIGLU>(p, nrt, st);
       rc = CWEN_OK;
     } else if (nsides == 1 && epi == GEMV_EPI_CONV) {
-      if (!out.cv_w || !out.cv_H || !out.cv_xc || !out.cv_ctl || out.cv_C < 0 || out.cv_C > w->ne1 || out.cv_C % Q4_ROWS ||
-          out.cv_nslot < 1)
-        return CWEN_EINVAL;
       launch_cb<GEMV_Q4, 1, GEMV_EPI_CONV>(p, nrt, st);
       rc = CWEN_OK;
     } else {

@@ -1,6 +1,8 @@
 // Super-tile layouts and their dequantisation to f16 MFMA operands, shared by
 // the kernels that stream quantized weights (layouts: gemv.hip).
 #pragma once
+#include <type_traits>
+
 #include "cwen_internal.h"
 
 namespace {
@@ -159,6 +161,87 @@ __device__ __forceinline__ half2_t bcast_half(uint32_t w, bool hi) {
 __device__ __forceinline__ half2_t i8pair(uint32_t w, uint32_t magic, bool upper) {
   const uint32_t t = __builtin_amdgcn_perm(magic, w, upper ? 0x07030502u : 0x07010500u);
   return __builtin_bit_cast(half2_t, t) - h2c(1152.f);
+}
+
+
+constexpr int TILES = Q4_ST_TILES;  // tiles per round: one super-tile per stream
+// A per-lane buffer offset past any activation range: the load returns zeros.
+constexpr uint32_t kPastRange = 0xFFFFFFE0u;
+struct GemvParams {
+  const uint8_t *w;    // super-tiled weights, round-major: super-tile (st, rg, side) at ((st*nrg + rg)*nsw + side)
+  uint32_t wbytes;     // bytes of the tiled weights (buffer range)
+  int nsw;             // sides stored per super-tile position (1 or 2)
+  int side0;           // first side computed (NS == 1)
+  int M, nrg, nst;
+  // Workgroups [0, nsplit) each take one piece of a split row tile: piece
+  // i % S (rounds (i % S) * rps ..) of tile tile0 + i / S.  The others take
+  // whole row tiles 0, 1, ...
+  int nsplit, S, rps, tile0;
+  const _Float16 *xh;  // activations f16 [B][K]
+  uint32_t xbytes;     // buffer range of the activations: columns >= B read as zero
+  const float *xf;     // XN: f32 rows [c*xfs + k], converted to f16 while staging
+  int xfs;
+  // Post-scale (f16 operand w * x, x not yet normalised): output column c is
+  // multiplied by 1 / sqrt(sum_p pss[p][c] / K + eps).
+  const float *pss;
+  int pnpart;
+  float eps;
+  int K, B;
+  float *part;         // split-K partials
+  int ncu;             // compute units of the device
+  int *cnt;            // per split-tile arrival counters (zero between launches)
+  GemvOut out;
+};
+
+// 8 f32 activations -> 8 f16, rounded to nearest.
+__device__ __forceinline__ uint4 cvt8(const uint4 (&x)[2]) {
+  const float4 x0 = __builtin_bit_cast(float4, x[0]), x1 = __builtin_bit_cast(float4, x[1]);
+  const half2_t h0 = {(_Float16)x0.x, (_Float16)x0.y}, h1 = {(_Float16)x0.z, (_Float16)x0.w};
+  const half2_t h2 = {(_Float16)x1.x, (_Float16)x1.y}, h3 = {(_Float16)x1.z, (_Float16)x1.w};
+  return make_uint4(__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1),
+                    __builtin_bit_cast(uint32_t, h2), __builtin_bit_cast(uint32_t, h3));
+}
+
+// 1 / rms of a column from its npart partial sums of squares: lane l adds
+// partials l, l + 64, ... in order, then one DPP tree over the wave, so every
+// launch and every block size gets the same scale.  Loads past npart return
+// zeros.
+struct PostParts {
+  float v[CWEN_MAX_PARTS / 64];
+};
+__device__ __forceinline__ void post_load(PostParts &q, const float *pp, int npart, int lane) {
+  const __amdgpu_buffer_rsrc_t r = make_rsrc(pp, (uint32_t)npart * 4);
+#pragma unroll
+  for (int j = 0; j < CWEN_MAX_PARTS / 64; ++j)
+    q.v[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, lane * 4 + j * 256, 0, 0));
+}
+__device__ __forceinline__ float post_scale(const PostParts &q, float K, float eps) {
+  float t = q.v[0];
+#pragma unroll
+  for (int j = 1; j < CWEN_MAX_PARTS / 64; ++j) t += q.v[j];
+  return 1.f / sqrtf(sum64(t) / K + eps);
+}
+
+// GatedDeltaNet conv rows (CONV epilogue): lane (g, n) holds positions 4g ..
+// 4g+3 of channel `row`; positions 4g-3 .. 4g-1 come from lane (g-1, n), or
+// for g = 0 from the history slot the block starts from (h).
+__device__ __forceinline__ void conv_store(const GemvOut &o, floatx4_t res, const float (&h)[3], float4 w, int cur, int P,
+                                           int row, int lane, int g, int B, bool store) {
+  const float p1 = __shfl(res[1], lane - 16), p2 = __shfl(res[2], lane - 16), p3 = __shfl(res[3], lane - 16);
+  if (!store) return;
+  const size_t hf = (size_t)o.cv_C * 3;
+  const float a[7] = {g == 0 ? h[0] : p1, g == 0 ? h[1] : p2, g == 0 ? h[2] : p3, res[0], res[1], res[2], res[3]};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int b = g * 4 + e;
+    if (b >= B) continue;
+    const float x = conv4(a[e], a[e + 1], a[e + 2], a[e + 3], w);
+    o.cv_xc[((size_t)P * CWEN_BMAX + b) * o.cv_C + row] = silu_f(x);
+    float *hs = o.cv_H + (size_t)((cur + 1 + b) % o.cv_nslot) * hf + (size_t)row * 3;
+    hs[0] = a[e + 1];
+    hs[1] = a[e + 2];
+    hs[2] = a[e + 3];
+  }
 }
 
 }  // namespace

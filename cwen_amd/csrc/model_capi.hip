@@ -141,7 +141,7 @@ Rows rows_of(const cwen_model_cfg &c) {
 int check_cfg(const cwen_model_cfg *c) {
   if (!c || c->n_layers <= 0 || c->d_model <= 0 || c->d_ffn <= 0 || c->vocab <= 0) return CWEN_EINVAL;
   if (c->d_model % Q4_K_ALIGN || c->d_ffn % Q4_K_ALIGN) return CWEN_EINVAL;
-  if (c->d_model > 8192) return CWEN_EINVAL;  // <= CWEN_MAX_PARTS row-tile partials of the residual's sum of squares
+  if (c->d_model > 8192) return CWEN_EINVAL;  // <= CWEN_MAX_PARTS partials of the residual's sum of squares
   if (c->head_dim != 256 || c->n_head <= 0 || c->n_kv_head <= 0 || c->n_head % c->n_kv_head) return CWEN_EINVAL;
   // Attention takes every block size up to CWEN_BMAX: refused here rather than
   // part-way through a block.
@@ -292,7 +292,7 @@ int mtp_pass(cwen_model *m, int B, const int *toks, const float *hsrc, int hs, c
   o0.rflag = rflag;
   if ((rc = gemv_launch(ctx, m->mtp_eh, 1, 0, GEMV_EPI_STORE, m->cat, o0, B, st))) return rc;
   const Rows r = rows_of(c);
-  const GemvPost n1 = {m->ssq2, gemv_row_tiles(m->mtp_eh), c.rms_eps};
+  const GemvPost n1 = {m->ssq2, gemv_ssq_parts(m->mtp_eh), c.rms_eps};
   GemvOut o1 = {m->att, nullptr, nullptr, r.att, 0};
   if ((rc = gemv_launch(ctx, y.att_in, 1, 0, GEMV_EPI_STORE, m->xh2, o1, B, st, nullptr, &n1))) return rc;
   if ((rc = attention_launch(m->att, r.att, m->att + r.Qo2, m->att + r.Qo2 + r.Ko, r.att, y.q_norm, y.k_norm,
@@ -304,7 +304,7 @@ int mtp_pass(cwen_model *m, int B, const int *toks, const float *hsrc, int hs, c
   o5.nwh = y.post_norm;
   o5.rflag = rflag;
   if ((rc = gemv_launch(ctx, y.wo, 1, 0, GEMV_EPI_STORE, m->yh, o5, B, st))) return rc;
-  const GemvPost n2 = {m->ssq2, gemv_row_tiles(y.wo), c.rms_eps};
+  const GemvPost n2 = {m->ssq2, gemv_ssq_parts(y.wo), c.rms_eps};
   GemvOut f1 = {nullptr, nullptr, m->hh, 0, 0};
   f1.rflag = rflag;
   GemvOut f2 = {m->X2, nullptr, m->xh2, H, 1};
@@ -315,7 +315,7 @@ int mtp_pass(cwen_model *m, int B, const int *toks, const float *hsrc, int hs, c
       (rc = gemv_launch(ctx, y.ffn_down, 1, 0, GEMV_EPI_STORE, m->hh, f2, B, st)))
     return rc;
   if (head_t < 0) return CWEN_OK;
-  const GemvPost nh = {m->ssq2, gemv_row_tiles(y.ffn_down), c.rms_eps};
+  const GemvPost nh = {m->ssq2, gemv_ssq_parts(y.ffn_down), c.rms_eps};
   GemvOut o = {m->mlogits + (size_t)head_t * c.vocab, nullptr, nullptr, c.vocab, 0,
                {ctx->amax_keys, ctx->amax_cnt, m->toks, 0, m->mres + 4 * head_t}};
   return gemv_launch(ctx, m->head, 1, 0, GEMV_EPI_ARGMAX, m->xh2, o, 1, st, nullptr, &nh);
@@ -408,7 +408,7 @@ int block(cwen_model *m, int B, int mode, hipStream_t st, const int *toks = null
       if ((rc = gemv_launch(ctx, y.wo, 1, 0, GEMV_EPI_STORE, m->yh, o5, B, st))) return rc;
       wout = y.wo;
     }
-    const GemvPost n2 = {m->ssq, gemv_row_tiles(wout), c.rms_eps};
+    const GemvPost n2 = {m->ssq, gemv_ssq_parts(wout), c.rms_eps};
     GemvOut f1 = {nullptr, nullptr, m->hh, 0, 0};
     f1.rflag = rflag;
     GemvOut f2 = {m->X, nullptr, m->xh, H, 1};
@@ -418,7 +418,7 @@ int block(cwen_model *m, int B, int mode, hipStream_t st, const int *toks = null
     if ((rc = gemv_launch(ctx, y.ffn_gu, 2, 0, GEMV_EPI_SWIGLU, m->xh, f1, B, st, nullptr, &n2)) ||
         (rc = gemv_launch(ctx, y.ffn_down, 1, 0, GEMV_EPI_STORE, m->hh, f2, B, st)))
       return rc;
-    npart = gemv_row_tiles(y.ffn_down);
+    npart = gemv_ssq_parts(y.ffn_down);
     (void)I;
   }
   if (mode != MODE_FWD) {
@@ -491,12 +491,14 @@ int wide_alloc(cwen_model *m, int n) {
                      wide_partial_floats(y.linear ? y.lin_in : y.att_in, 1, false, N),
                      wide_partial_floats(y.linear ? y.ssm_out : y.wo, 1, true, N)});
   }
+  // The products read whole tiles of 64 positions, past the last one's end.
+  constexpr size_t kSlack = 64 * 128;
   int rc = (dmalloc(&m->wtoks, np) || dmalloc(&m->wX, np * H) || dmalloc(&m->wssq, np * CWEN_MAX_PARTS) ||
             dmalloc(&m->wpsc, np + 64) || dmalloc(&m->wlin, np * wide_ls(c)) || dmalloc(&m->wxc, np * R.C) ||
             dmalloc(&m->wgates, np * 2 * R.nvh) || dmalloc(&m->wq, np * Qo) || dmalloc(&m->wpart, part) ||
             dmalloc(&m->watt, att) ||
-            dmalloc(&m->wxh, np * H) || dmalloc(&m->wgh, np * std::max((size_t)R.Zh, Qo)) ||
-            dmalloc(&m->whh, np * c.d_ffn) ||
+            dmalloc(&m->wxh, np * H + kSlack) || dmalloc(&m->wgh, np * std::max((size_t)R.Zh, Qo) + kSlack) ||
+            dmalloc(&m->whh, np * c.d_ffn + kSlack) ||
             hipHostMalloc((void **)&m->hwtok, np * sizeof(int), hipHostMallocDefault) != hipSuccess)
                ? CWEN_ENOMEM
                : CWEN_OK;
@@ -545,14 +547,14 @@ int wide_block(cwen_model *m, int N, hipStream_t st) {
     const cwen_weight *wout = y.linear ? y.ssm_out : y.wo;
     const WideOut oo = {m->wX, H, 1, m->wxh, y.post_norm, m->wssq, rflag};
     if ((rc = wide_gemm(ctx, wout, GEMV_EPI_STORE, m->wgh, N, nullptr, oo, m->wpart, st)) ||
-        (rc = wide_scale(m->wssq, gemv_row_tiles(wout), H, c.rms_eps, N, m->wpsc, st)))
+        (rc = wide_scale(m->wssq, gemv_ssq_parts(wout), H, c.rms_eps, N, m->wpsc, st)))
       return rc;
     const WideOut of = {nullptr, 0, 0, m->whh, nullptr, nullptr, rflag};
     const WideOut od = {m->wX, H, 1, m->wxh, l + 1 < c.n_layers ? m->L[l + 1].attn_norm : m->out_norm, m->wssq, rflag};
     if ((rc = wide_gemm(ctx, y.ffn_gu, GEMV_EPI_SWIGLU, m->wxh, N, m->wpsc, of, m->wpart, st)) ||
         (rc = wide_gemm(ctx, y.ffn_down, GEMV_EPI_STORE, m->whh, N, nullptr, od, m->wpart, st)))
       return rc;
-    npart = gemv_row_tiles(y.ffn_down);
+    npart = gemv_ssq_parts(y.ffn_down);
   }
   hipLaunchKernelGGL(wide_advance_kernel, dim3(1), dim3(1), 0, st, m->ctl, N, CWEN_BMAX + 1);
   CWEN_HIP_TRY(hipGetLastError());

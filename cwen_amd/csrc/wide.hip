@@ -38,6 +38,7 @@ namespace {
 constexpr int WW = 4;                // waves per workgroup
 constexpr int TG = 4;                // row groups of a single-sided row tile of gemv_kernel
 
+
 struct WideParams {
   const uint8_t *w;
   uint32_t wbytes;
@@ -307,11 +308,11 @@ __global__ __launch_bounds__(256) void wide_finish_kernel(WideParams p, WideOut 
         o.yh[wide_at(c, row, p.N)] = h;
         if (f16_bad(h)) raise_flag(p.rflag);
       }
-      sq = r * r;
+      sq = f32_of(r * r);
     }
     if (o.ssq) {
-      sq = sum64(sq);
-      if (lane == 0) o.ssq[(size_t)c * CWEN_MAX_PARTS + row / 64] = sq;
+      sq = sum16(sq);
+      if ((lane & 15) == 0 && ok) o.ssq[(size_t)c * CWEN_MAX_PARTS + row / 16] = sq;
     }
   }
 }
@@ -321,10 +322,9 @@ __global__ __launch_bounds__(256) void wide_finish_kernel(WideParams p, WideOut 
 __global__ __launch_bounds__(256) void wide_scale_kernel(const float *ssq, int npart, int K, float eps, int N, float *psc) {
   const int lane = threadIdx.x & 63, c = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (c >= N) return;
-  const float *pp = ssq + (size_t)c * CWEN_MAX_PARTS;
-  float v = lane < npart ? pp[lane] : 0.f;
-  if (lane + 64 < npart) v += pp[lane + 64];
-  const float s = 1.f / sqrtf(sum64(v) / (float)K + eps);
+  PostParts q;
+  post_load(q, ssq + (size_t)c * CWEN_MAX_PARTS, npart, lane);
+  const float s = post_scale(q, (float)K, eps);
   if (lane == 0) psc[c] = s;
 }
 

@@ -357,3 +357,60 @@ def test_elementwise_error_bound(env, kind, K):
         assert (r <= 1).all(), (kind, K, B, float(r.max()))
         worst = max(worst, float(r.max()))
     print(f"{kind} K={K}: worst error / bound {worst:.3f}")
+
+
+# Weights small enough for K to be split over a workgroup's waves: one wave and
+# one round; rows and K ragged; the most pieces; a wave with 3 rounds and one
+# shorter; more row groups than CUs (two row groups per wave at B > 4, the last
+# one alone, activations staged or converted first); sizes just past each limit
+# (15 rounds at more row groups than CUs, 6 rounds a wave).
+KW_SHAPES = [(16, 32), (17, 480), (100, 2080), (1000, 3072), (4096, 8704), (4100, 2592), (8192, 544), (4300, 7680),
+             (64, 17408)]
+
+
+@pytest.mark.parametrize("M,K", KW_SHAPES)
+def test_split_in_workgroup(env, oracle, M, K):
+    """f32 and f16 entry points against the oracle, block invariance bit for
+    bit over both, accumulation onto a residual and the f16 copy."""
+    torch, gpu, ctx = env
+    print(f"split in workgroup {M}x{K}", flush=True)
+    qs, sc = synth.q4_rs(130, M, K)
+    W = gpu.Weight(ctx, T_RS, qs, sc, K, M)
+    X = synth.activations(130, 16, K)
+    want = oracle.gemvb(T_RS, qs, sc, K, M, X)
+    full = _run(env, W, X)
+    assert rel_err(full, want) <= TOL
+    for B in (1, 2, 3, 4, 5, 8, 9):
+        assert np.array_equal(_run(env, W, X[:B]).view(np.uint32), full[:B].view(np.uint32)), B
+    Xh = torch.from_numpy(X).cuda().half()
+    Y0 = torch.from_numpy(synth.activations(131, 16, M)).cuda()
+    for B in (1, 4, 7, 16):
+        Y, Yh = Y0[:B].clone(), torch.zeros(B, M, dtype=torch.float16, device="cuda")
+        if M % 8 == 0:
+            gpu.gemvb_f16(ctx, W, Xh, Y, B, Yh=Yh, accumulate=True)
+            torch.cuda.synchronize()
+            assert torch.equal(Yh, Y.half())
+        else:
+            gpu.gemvb_f16(ctx, W, Xh, Y, B, accumulate=True)
+            torch.cuda.synchronize()
+        assert np.array_equal(Y.cpu().numpy(), (Y0[:B].cpu().numpy() + full[:B])), B
+
+
+@pytest.mark.parametrize("M,K", [(40, 96), (1024, 5120), (4096, 1024), (4112, 1024)])
+def test_split_in_workgroup_pairs(env, oracle, M, K):
+    """Pair, single sides and SwiGLU of small pairs, every block size class."""
+    torch, gpu, ctx = env
+    print(f"split in workgroup, pair {M}x{K}", flush=True)
+    qs, sc = synth.q4_rsi(132, M, K)
+    W = gpu.Weight(ctx, T_RSI, qs, sc, K, M)
+    X = synth.activations(132, 16, K)
+    wa, wb = (oracle.gemvb(T_RSI, qs, sc, K, M, X, side=s) for s in (0, 1))
+    ya, yb = _run(env, W, X, mode="pair")
+    assert rel_err(ya, wa) <= TOL and rel_err(yb, wb) <= TOL
+    h = _run(env, W, X, mode="swiglu")
+    assert rel_err(h, oracle.silu_mul(wa, wb)) <= TOL
+    for B in (1, 3, 5, 9):
+        pa, pb = _run(env, W, X[:B], mode="pair")
+        assert np.array_equal(pa, ya[:B]) and np.array_equal(pb, yb[:B]), B
+        assert np.array_equal(_run(env, W, X[:B], side=1), yb[:B]), B
+        assert np.array_equal(_run(env, W, X[:B], mode="swiglu"), h[:B]), B
