@@ -291,14 +291,16 @@ static int check_w(const cwen_ctx *ctx, const cwen_weight *W) {
 // workgroups (small weights) the launch saved is the larger, up to B = 8 or
 // while there are no more row groups than CUs: 1000 x 2080 at B = 16 5.1 us staged,
 // 7.7 converted first; 5120 x 5120 11.4 and 11.1.
+// Columns further apart than a buffer's 32-bit byte range are always converted first.
 // nsides 0: the head's launch, always whole rows.
-static bool f32_staged(const cwen_weight *W, int nsides, int B) {
+static bool f32_staged(const cwen_weight *W, int nsides, int xs, int B) {
+  if (((uint64_t)(B - 1) * xs + W->ne0) * 4 > UINT32_MAX - 64) return false;
   const bool kw = nsides && W->cfg[nsides - 1].kw;
   return B <= (!kw ? 4 : W->nrg > W->ctx->ncu ? 8 : CWEN_BMAX);
 }
 static int f32_operand(cwen_ctx *ctx, const cwen_weight *W, int nsides, const float *X, int xs, int B, hipStream_t st,
                        GemvF32 *n, const _Float16 **xh) {
-  if (f32_staged(W, nsides, B)) {
+  if (f32_staged(W, nsides, xs, B)) {
     *n = {X, xs};
     *xh = nullptr;
     return CWEN_OK;
@@ -419,7 +421,7 @@ int cwen_mlp_block_noalloc(const cwen_weight *Wgu, const cwen_weight *Wd, const 
   hipStream_t st = (hipStream_t)stream;
   _Float16 *const xh = (_Float16 *)(base + kStaticXhOfs), *const hh = (_Float16 *)(base + kStaticHhOfs);
   GemvF32 x = {X, xs};
-  const bool stage_f32 = f32_staged(Wgu, 2, B);  // the GEMV converts X while staging (cwen_mlp_block's rule)
+  const bool stage_f32 = f32_staged(Wgu, 2, xs, B);  // the GEMV converts X while staging (cwen_mlp_block's rule)
   if (!stage_f32 && (rc = act_to_f16(X, xs, xh, Wgu->ne0, B, st))) return rc;
   GemvOut o1 = {nullptr, nullptr, hh, 0, 0};
   if ((rc = gemv_launch(ctx, Wgu, 2, 0, GEMV_EPI_SWIGLU, stage_f32 ? nullptr : xh, o1, B, st,

@@ -45,7 +45,9 @@
 //    depends on activation column c alone, so the unstaged columns only feed
 //    discarded outputs, and a column's arithmetic never depends on B (block
 //    verify == serial decode, bit for bit).
-//  * Long K is split across workgroups.  Each writes its partial sums with
+//  * Long K of small weights is split over the waves of a workgroup
+//    (gemv_kw.hip; choose_grid draws the line), of larger ones across
+//    workgroups.  There each writes its partial sums with
 //    agent-scope atomic stores, bumps a per-row-tile counter, and the last
 //    arriver sums the partials in split order: deterministic, with no cache
 //    writeback/invalidate.  The split depends on the shape only.

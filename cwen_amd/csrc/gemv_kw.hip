@@ -21,7 +21,15 @@ constexpr int KW_MAX = GEMV_KW_MAX;   // pieces of K at most
 // barrier in the loop, and keeps one round of weights in flight while it
 // computes another.  The residual, the norm weight and the conv's history are
 // requested before the loop.
-// Measured (27B shapes, before -> after): NNN
+// Measured against the split over workgroups (us, f16 / f32 activations of the
+// caller; medians):
+//   Q4_0 1000 x 2080  B = 1   6.5 -> 4.4        Q4_0 2048 x 6144  B = 4  7.4 -> 5.2
+//   Q4_0 5120 x 5120  B = 1   8.0 -> 7.05       Q8_0 3001 x 4128  B = 5  9.3 -> 6.4
+//   Q4_0 5120 x 6144  B = 1, 2, 3, 4, f32       8.6, 8.8, 8.9, 9.4 before
+//                                               7.4, 8.0, 8.9, 9.4 now
+//   k/v pair 1024 x 5120  B = 16  9.1 -> 7.1    FFN 2048 x 5632  B = 16  17.1 -> 15.7
+// What is left at these sizes is the launch, one round trip to memory for the
+// first round of weights and one for the sums: 2-3 us before the first MFMA.
 template <int FMT, int NS, int EPI, int CB, bool XN, int RGW>
 __global__ __launch_bounds__(64 * KW_MAX * NS) void gemv_kw_kernel(GemvParams p) {
   using F = Fmt<FMT>;
@@ -61,27 +69,29 @@ __global__ __launch_bounds__(64 * KW_MAX * NS) void gemv_kw_kernel(GemvParams p)
   };
   auto load_round = [&](Round (&ws)[RGW], int r) __attribute__((always_inline)) {
 #pragma unroll
-   for (int k = 0; k < RGW; ++k) {
-    Round &w = ws[k];
-    const uint32_t so = wofs[k] + (uint32_t)r * sstride;
-    if constexpr (DM) w.sc = bload16_nt(wr, F::SC_OFS + lane * 16, so);
-    else w.sc = bload8_nt(wr, F::SC_OFS + lane * 8, so);
-    if constexpr (FMT == GEMV_Q6K) w.dq = bload4_nt(wr, F::D_OFS + n * 4, so);
-    if constexpr (FMT == GEMV_Q5K) w.h5 = bload16_nt(wr, F::HI_OFS + lane * 16, so);
+    for (int k = 0; k < RGW; ++k) {
+      Round &w = ws[k];
+      const uint32_t so = wofs[k] + (uint32_t)r * sstride;
+      if constexpr (DM) w.sc = bload16_nt(wr, F::SC_OFS + lane * 16, so);
+      else w.sc = bload8_nt(wr, F::SC_OFS + lane * 8, so);
+      if constexpr (FMT == GEMV_Q6K) w.dq = bload4_nt(wr, F::D_OFS + n * 4, so);
+      if constexpr (FMT == GEMV_Q5K) w.h5 = bload16_nt(wr, F::HI_OFS + lane * 16, so);
 #pragma unroll
-    for (int t = 0; t < TILES; ++t) {
+      for (int t = 0; t < TILES; ++t) {
 #pragma unroll
-      for (int v = 0; v < TV; ++v) w.q[t][v] = bload16_nt(wr, lane * 16 + t * (1024 * TV) + v * 1024, so);
-      if constexpr (FMT == GEMV_Q6K) {
-        if (t & 1) w.hq[t >> 1] = bload16_nt(wr, F::HI_OFS + (t >> 1) * 1024 + lane * 16, so);
+        for (int v = 0; v < TV; ++v) w.q[t][v] = bload16_nt(wr, lane * 16 + t * (1024 * TV) + v * 1024, so);
+        if constexpr (FMT == GEMV_Q6K) {
+          if (t & 1) w.hq[t >> 1] = bload16_nt(wr, F::HI_OFS + (t >> 1) * 1024 + lane * 16, so);
+        }
       }
     }
-   }
   };
   // Activations of half round h: lane (c2, u) of load i takes unit u (8 K) of
   // column 2 i + c2.  LDS unit c * 32 + (u' ^ (c & 15)), u' = u with bits 2-3
   // negated (see wide.hip: 16-byte reads without bank conflicts).  Units past K
-  // and columns past B read as zeros.
+  // and columns past B read as zeros.  The LDS is this wave's own and served in
+  // order; wave_fence keeps the compiler from moving a lane's reads past the
+  // writes that other lanes made for it.
   const int xc = lane >> 5, xu = lane & 31;
   const int xp = (xu & 16) | (((4 - ((xu >> 2) & 3)) & 3) << 2) | (xu & 3);
   constexpr int XL = CB / 2;                   // staging loads per half round (two columns each)
@@ -104,6 +114,11 @@ __global__ __launch_bounds__(64 * KW_MAX * NS) void gemv_kw_kernel(GemvParams p)
       if constexpr (XN) act[c * HU + (xp ^ (c & 15))] = cvt8(xs[i]);
       else act[c * HU + (xp ^ (c & 15))] = xs[i][0];
     }
+  };
+
+  auto wave_fence = []() __attribute__((always_inline)) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
   };
 
   stage_load(0);
@@ -162,7 +177,9 @@ __global__ __launch_bounds__(64 * KW_MAX * NS) void gemv_kw_kernel(GemvParams p)
     if (rd + 1 < nround) load_round(next, rd + 1);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      wave_fence();
       stage_store();
+      wave_fence();
       if (2 * rd + h + 1 < 2 * nround) stage_load(2 * rd + h + 1);
 #pragma unroll
       for (int t = 2 * h; t < 2 * h + 2; ++t) {

@@ -151,6 +151,26 @@ def test_strided_activations_and_outputs(env, oracle):
     assert np.all(Yh[:, M:] == 7.0)  # nothing written past M
 
 
+@pytest.mark.parametrize("B,xs", [(5, 1 << 28), (3, 1 << 29)])
+def test_columns_past_32_bits_of_bytes(env, B, xs):
+    """Columns whose byte offsets pass 2^32, as the contiguous ones, bit for bit."""
+    torch, gpu, ctx = env
+    M, K = 96, 512
+    qs, sc = synth.q4_rs(109, M, K)
+    W = gpu.Weight(ctx, T_RS, qs, sc, K, M)
+    X = torch.from_numpy(synth.activations(109, B, K)).cuda()
+    Xd = torch.empty((B - 1) * xs + K, device="cuda")
+    for b in range(B):
+        Xd[b * xs:b * xs + K] = X[b]
+    want, got = torch.zeros(B, M, device="cuda"), torch.zeros(B, M, device="cuda")
+    gpu.gemvb(ctx, W, X, want, B)
+    gpu.gemvb(ctx, W, Xd, got, B, xs=xs)
+    torch.cuda.synchronize()
+    del Xd
+    torch.cuda.empty_cache()
+    assert torch.equal(want, got)
+
+
 def test_argument_errors(env):
     torch, gpu, ctx = env
     M, K = 32, 512
