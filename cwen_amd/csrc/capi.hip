@@ -290,17 +290,17 @@ static int check_w(const cwen_ctx *ctx, const cwen_weight *W) {
 // every workgroup of the GEMV), measured on the FFN shapes.  With K split inside the
 // workgroups (small weights) the launch saved is the larger, up to B = 8 or
 // while there are no more row groups than CUs: 1000 x 2080 at B = 16 5.1 us staged,
-// 7.7 converted first; 5120 x 5120 11.4 and 11.1.
+// 7.7 converted first; 5120 x 5120 11.4 and 11.1; SwiGLU 2048 x 3072 11.4 and 9.4.
 // Columns further apart than a buffer's 32-bit byte range are always converted first.
-// nsides 0: the head's launch, always whole rows.
-static bool f32_staged(const cwen_weight *W, int nsides, int xs, int B) {
+// form: the launch's entry of W->cfg; -1: the head's launch, always whole rows.
+static bool f32_staged(const cwen_weight *W, int form, int xs, int B) {
   if (((uint64_t)(B - 1) * xs + W->ne0) * 4 > UINT32_MAX - 64) return false;
-  const bool kw = nsides && W->cfg[nsides - 1].kw;
-  return B <= (!kw ? 4 : W->nrg > W->ctx->ncu ? 8 : CWEN_BMAX);
+  const bool kw = form >= 0 && W->cfg[form].kw;
+  return B <= (!kw ? 4 : form == 1 || W->nrg > W->ctx->ncu ? 8 : CWEN_BMAX);
 }
-static int f32_operand(cwen_ctx *ctx, const cwen_weight *W, int nsides, const float *X, int xs, int B, hipStream_t st,
+static int f32_operand(cwen_ctx *ctx, const cwen_weight *W, int form, const float *X, int xs, int B, hipStream_t st,
                        GemvF32 *n, const _Float16 **xh) {
-  if (f32_staged(W, nsides, xs, B)) {
+  if (f32_staged(W, form, xs, B)) {
     *n = {X, xs};
     *xh = nullptr;
     return CWEN_OK;
@@ -325,7 +325,7 @@ int cwen_gemvb(cwen_ctx *ctx, const cwen_weight *W, int side, const float *X, in
   hipStream_t st = (hipStream_t)stream;
   GemvF32 x;
   const _Float16 *xh;
-  if ((rc = f32_operand(ctx, W, 1, X, xs, B, st, &x, &xh))) return rc;
+  if ((rc = f32_operand(ctx, W, 0, X, xs, B, st, &x, &xh))) return rc;
   GemvOut o = {Y, nullptr, nullptr, ys, 0};
   return gemv_launch(ctx, W, 1, side, GEMV_EPI_STORE, xh, o, B, st, xh ? nullptr : &x);
 }
@@ -341,7 +341,7 @@ int cwen_gemvb_pair(cwen_ctx *ctx, const cwen_weight *W, const float *X, int xs,
   hipStream_t st = (hipStream_t)stream;
   GemvF32 x;
   const _Float16 *xh;
-  if ((rc = f32_operand(ctx, W, W->cfg[0].kw ? 1 : 2, X, xs, B, st, &x, &xh))) return rc;
+  if ((rc = f32_operand(ctx, W, 2, X, xs, B, st, &x, &xh))) return rc;
   GemvOut o = {YA, YB, nullptr, ys, 0};
   return gemv_launch(ctx, W, 2, 0, GEMV_EPI_PAIR, xh, o, B, st, xh ? nullptr : &x);
 }
@@ -355,7 +355,7 @@ int cwen_gemvb_swiglu(cwen_ctx *ctx, const cwen_weight *W, const float *X, int x
   hipStream_t st = (hipStream_t)stream;
   GemvF32 x;
   const _Float16 *xh;
-  if ((rc = f32_operand(ctx, W, 2, X, xs, B, st, &x, &xh))) return rc;
+  if ((rc = f32_operand(ctx, W, 1, X, xs, B, st, &x, &xh))) return rc;
   GemvOut o = {H, nullptr, nullptr, hs, 0};
   return gemv_launch(ctx, W, 2, 0, GEMV_EPI_SWIGLU, xh, o, B, st, xh ? nullptr : &x);
 }
@@ -394,7 +394,7 @@ int cwen_mlp_block(cwen_ctx *ctx, const cwen_weight *Wgu, const cwen_weight *Wd,
   hipStream_t st = (hipStream_t)stream;
   GemvF32 x;
   const _Float16 *xh;
-  if ((rc = f32_operand(ctx, Wgu, 2, X, xs, B, st, &x, &xh))) return rc;
+  if ((rc = f32_operand(ctx, Wgu, 1, X, xs, B, st, &x, &xh))) return rc;
   GemvOut o1 = {nullptr, nullptr, ctx->hh, 0, 0};
   if ((rc = gemv_launch(ctx, Wgu, 2, 0, GEMV_EPI_SWIGLU, xh, o1, B, st, xh ? nullptr : &x))) return rc;
   GemvOut o2 = {Y, nullptr, nullptr, ys, 1};
@@ -421,7 +421,7 @@ int cwen_mlp_block_noalloc(const cwen_weight *Wgu, const cwen_weight *Wd, const 
   hipStream_t st = (hipStream_t)stream;
   _Float16 *const xh = (_Float16 *)(base + kStaticXhOfs), *const hh = (_Float16 *)(base + kStaticHhOfs);
   GemvF32 x = {X, xs};
-  const bool stage_f32 = f32_staged(Wgu, 2, xs, B);  // the GEMV converts X while staging (cwen_mlp_block's rule)
+  const bool stage_f32 = f32_staged(Wgu, 1, xs, B);  // the GEMV converts X while staging (cwen_mlp_block's rule)
   if (!stage_f32 && (rc = act_to_f16(X, xs, xh, Wgu->ne0, B, st))) return rc;
   GemvOut o1 = {nullptr, nullptr, hh, 0, 0};
   if ((rc = gemv_launch(ctx, Wgu, 2, 0, GEMV_EPI_SWIGLU, stage_f32 ? nullptr : xh, o1, B, st,
@@ -442,7 +442,7 @@ int cwen_head_verify(cwen_ctx *ctx, const cwen_weight *W, const float *X, int xs
   hipStream_t st = (hipStream_t)stream;
   GemvF32 x;
   const _Float16 *xh;
-  if ((rc = f32_operand(ctx, W, 0, X, xs, B, st, &x, &xh))) return rc;
+  if ((rc = f32_operand(ctx, W, -1, X, xs, B, st, &x, &xh))) return rc;
   GemvOut o = {logits, nullptr, nullptr, ls, 0, {ctx->amax_keys, ctx->amax_cnt, drafts, E, res}};
   return gemv_launch(ctx, W, 1, 0, GEMV_EPI_ARGMAX, xh, o, B, st, xh ? nullptr : &x);
 }

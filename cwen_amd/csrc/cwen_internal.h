@@ -57,7 +57,7 @@ struct cwen_weight {
   uint8_t *dev;             // tiled device data
   size_t bytes;             // device bytes of the tiled data
   size_t src_bytes;         // bytes of the reference layout (qs + scales)
-  GemvGrid cfg[2];          // decomposition for one side / both sides of a pair (shape-only); PAIR: see gemv_launch
+  GemvGrid cfg[3];          // decomposition for one side / SwiGLU / both sides of a pair (shape-only)
   int rows;                 // row groups per wave (shape-only)
 };
 

@@ -975,11 +975,13 @@ double grid_cost(int ncu, int nst, const GemvGrid &c, double extra) {
 // Small weights (kw): K split over the waves of a workgroup per row group, for
 // about 7 waves per CU, when tiles are at most half as many as CUs, a wave gets
 // at most 3 rounds and the weight has at most 18 MB.  With more row groups than
-// CUs, some of which then run two workgroups, at most 2 rounds and, unless Q4_0, 14
-// MB: 4300 x 7680 (269 groups, 3 rounds) 8.9-11.9 against 9.0-10.3, Q4_1 5120 x 5120
+// CUs, some of which then run two workgroups, at most 2 rounds of at most 10 and,
+// unless Q4_0, 14 MB: 5120 x 6144 (12 rounds, f32, B = 1 / 4 / 16) 8.7 / 10.0 / 11.5 against
+// 8.4 / 8.5 / 11.2 us, 4300 x 7680 (269 groups, 3 rounds) 8.9-11.9 against 9.0-10.3, Q4_1 5120 x 5120
 // f32 at B = 4 9.1 against 8.2 us.  Measured against the forms below, f16 in, B = 1 / 4 /
-// 8 / 16: 5120 x 6144 (3840 super-tiles, 2 rounds) 7.3 / 8.3 / 8.9 / 9.3 against 8.6 / 8.8 / 8.9
-// / 9.4 us, 2048 x 6144 5.1 / 5.8 / 6.1 / 6.9 against 7.4 / 7.6 / 7.7 / 8.0,
+// 8 / 16: 5120 x 5120 7.1 / 7.6 / 8.5 / 9.1 against 8.3 / 8.5 / 8.6 / 9.1 us, 8000 x 2048
+// 4.6 / 4.8 / 4.8 / 5.3 against 6.9 / 7.2 / 7.3 / 8.0, 2048 x 6144 5.1 / 5.8 / 6.1 / 6.9 against
+// 7.4 / 7.6 / 7.7 / 8.0,
 // 1000 x 2080 4.5 / 4.5 / 4.6 / 4.8 against 6.6 / 7.1 / 7.1 / 7.5.  Past it a wave's own
 // activation staging shows: 5120 x 17408 (6 rounds) 15.6 / 17.2 / 19.7 / 26.6
 // against 13.8 / 14.1 / 14.7 / 15.6, Q5_K 5120 x 6144 (23.6 MB) 9.2 / 9.9 / 10.5 /
@@ -993,15 +995,21 @@ double grid_cost(int ncu, int nst, const GemvGrid &c, double extra) {
 // length.
 // split_basis: the tile count that sizes the split (the single-side one for
 // both launch kinds, so a pair launch splits K as its single sides do); bytes:
-// of one side; kw: allowed (a SwiGLU launch puts both sides into one workgroup: at 352
-// row groups x 4 rounds, B = 16, 9.0 us against 8.0 in whole tiles).
+// of one side; kw: allowed.  It is for single weights; for interleaved pairs while
+// both sides' row groups fit the CUs (pair launch, f32, B = 1 / 4 / 16: 1024 x 5120
+// 5.4 / 5.8 / 7.4 against 6.8 / 6.9 / 9.4 us, 2048 x 6144 6.3 / 6.7 / 9.4 against 8.4 / 8.5 /
+// 11.3, but 6144 x 4096 8.3 / 9.6 / 13.0 against 8.9 / 8.9 / 11.7); for SwiGLU, whose
+// workgroups hold both sides, up to one row group per CU and 6 rounds (f16 activations,
+// B = 1 / 4 / 16: 2048 x 3072 5.1 / 5.8 / 6.8 against 7.0 / 7.1 / 7.4 us, but 1408 x 4096 5.6 /
+// 6.2 / 8.1 against 6.9 / 7.0 / 7.3 and, at 352 row groups x 4 rounds, 9.0 against 8.0
+// in whole tiles at B = 16).
 GemvGrid choose_grid(const cwen_ctx *ctx, int ntile, int nst, int split_basis, int nrg, size_t bytes, int fmt, bool kw) {
   GemvGrid best = {ntile, 0, 1, nst, 0, 0};
   if (kw && 2 * split_basis <= ctx->ncu && bytes <= (size_t)18 << 20) {
-    const int S0 = std::min({std::max(7 * ctx->ncu / nrg, 1), GEMV_KW_MAX, nst});
+    const int S0 = std::min({std::max((7 * ctx->ncu + nrg / 2) / nrg, 1), GEMV_KW_MAX, nst});
     const int rps = (nst + S0 - 1) / S0, S = (nst + rps - 1) / rps;
     const bool one_wave_of_groups = nrg <= ctx->ncu;
-    if (one_wave_of_groups ? rps <= 3 : rps <= 2 && (fmt == GEMV_Q4 || bytes <= (size_t)14 << 20))
+    if (one_wave_of_groups ? rps <= 3 : rps <= 2 && nst <= 10 && (fmt == GEMV_Q4 || bytes <= (size_t)14 << 20))
       return {ntile * S, ntile * S, S, rps, 0, 1};
   }
   // More than half as many tiles as CUs: whole tiles, one per CU.  Split in
@@ -1044,11 +1052,23 @@ GemvGrid choose_grid(const cwen_ctx *ctx, int ntile, int nst, int split_basis, i
 void gemv_choose_split(const cwen_ctx *ctx, cwen_weight *w) {
   w->rows = 1;
   const int single = (w->nrg + tile_rows(1) - 1) / tile_rows(1);
-  for (int ns = 1; ns <= w->nside; ++ns) {
+  auto grid = [&](int ns, bool kw) {
     const int rpw = tile_rows(ns);
-    w->cfg[ns - 1] = choose_grid(ctx, (w->nrg + rpw - 1) / rpw, w->nst, single, w->nrg, w->bytes / w->nside, w->fmt,
-                                 ns == 1 || w->nrg <= ctx->ncu);
-  }
+    return choose_grid(ctx, (w->nrg + rpw - 1) / rpw, w->nst, single, w->nrg, w->bytes / w->nside, w->fmt, kw);
+  };
+  w->cfg[0] = grid(1, w->nside == 1 || 2 * w->nrg <= ctx->ncu);
+  if (w->nside == 1) return;
+  w->cfg[1] = grid(2, w->nrg <= ctx->ncu && w->nst <= 6);
+  w->cfg[2] = w->cfg[0].kw ? w->cfg[0] : grid(2, false);   // inside workgroups the sides are launched side by side
+}
+
+// A weight split inside workgroups whose launch takes the same pieces across
+// workgroups instead (the same sums in the same order): with more row groups than
+// CUs a CU's two workgroups stage the same activations, and from 9 rounds on that
+// shows for f32 ones at B = 3-4.  Inside / across, us: 5120 x 5120 at B = 4 8.5 /
+// 8.25, B = 3 8.2 / 8.2, B = 1 7.5 / 8.2; 6144 x 4096 (8 rounds) at B = 4 7.1 / 8.2.
+static bool kw_across(const cwen_ctx *ctx, const cwen_weight *w, bool f32, int B) {
+  return w->nrg > ctx->ncu && w->nst > 8 && f32 && (B == 3 || B == 4);
 }
 
 int gemv_ssq_parts(const cwen_weight *w) { return w->nrg; }
@@ -1068,8 +1088,7 @@ int gemv_launch(cwen_ctx *ctx, const cwen_weight *w, int nsides, int side0, int 
   p.M = w->ne1;
   p.nrg = w->nrg;
   p.nst = w->nst;
-  // A pair's two sides with K split inside workgroups are launched side by side.
-  GemvGrid cfg = w->cfg[epi == GEMV_EPI_PAIR && w->cfg[0].kw ? 0 : nsides - 1];
+  GemvGrid cfg = w->cfg[epi == GEMV_EPI_PAIR ? 2 : nsides - 1];
   p.xh = xh;
   const int xfs = xf ? (B > 1 ? xf->xs : w->ne0) : 0;
   p.xbytes = xf ? (uint32_t)(((size_t)(B - 1) * xfs + w->ne0) * 4) : (uint32_t)((size_t)B * w->ne0 * 2);
@@ -1087,6 +1106,10 @@ int gemv_launch(cwen_ctx *ctx, const cwen_weight *w, int nsides, int side0, int 
   const int rpw = tile_rows(nsides);
   const int ntile = (w->nrg + rpw - 1) / rpw;
   if (epi == GEMV_EPI_ARGMAX) cfg = {ntile, 0, 1, w->nst, 0, 0};  // final row values in one workgroup
+  if (cfg.kw && cfg.S > 1 && nsides == 1 && kw_across(ctx, w, xf != nullptr, B)) {
+    const GemvGrid a = {ntile * cfg.S, ntile * cfg.S, cfg.S, cfg.rps, 0, 0};
+    if (gemv_grid_fits(a, scr ? scr->partials_floats : ctx->partials_floats, scr ? scr->ncounters : ctx->ncounters)) cfg = a;
+  }
   if (scr && !gemv_grid_fits(cfg, scr->partials_floats, scr->ncounters)) return CWEN_ESCRATCH;
   p.nsplit = cfg.nsplit;
   p.S = cfg.S;

@@ -25,8 +25,7 @@ constexpr int KW_MAX = GEMV_KW_MAX;   // pieces of K at most
 // caller; medians):
 //   Q4_0 1000 x 2080  B = 1   6.5 -> 4.4        Q4_0 2048 x 6144  B = 4  7.4 -> 5.2
 //   Q4_0 5120 x 5120  B = 1   8.0 -> 7.05       Q8_0 3001 x 4128  B = 5  9.3 -> 6.4
-//   Q4_0 5120 x 6144  B = 1, 2, 3, 4, f32       8.6, 8.8, 8.9, 9.4 before
-//                                               7.4, 8.0, 8.9, 9.4 now
+//   Q4_0 8000 x 2048  B = 4   7.2 -> 4.8        Q4_0 6144 x 4096  B = 16 9.0 -> 7.2
 //   k/v pair 1024 x 5120  B = 16  9.1 -> 7.1    FFN 2048 x 5632  B = 16  17.1 -> 15.7
 // What is left at these sizes is the launch, one round trip to memory for the
 // first round of weights and one for the sums: 2-3 us before the first MFMA.
@@ -296,10 +295,9 @@ int launch_one(const GemvParams &p, hipStream_t st) {
   const dim3 block(64u * nwave), grid1((unsigned)p.nrg, EPI == GEMV_EPI_PAIR ? 2u : 1u);
   static_assert(CB * NS <= 16 || (FMT == GEMV_Q4 && NS == 2 && CB == 16), "LDS above 64 KB: see gemv_kw_init");
   // Wide blocks over more row groups than CUs: two row groups per wave, which
-  // share its staged activations.  5120 x 6144 (320 row groups): at B = 16 9.3
-  // against 10.6 us with one, f32 activations at B = 8 9.6 against 10.6 (5120 x
-  // 5120, f16: 8.4 against 8.2-9.8, unsteady); at B <= 4 the halved workgroup
-  // count costs more (8.2 against 7.3 us at B = 1), except for f32 activations
+  // share its staged activations (5120 x 5120, f16, B = 16: 8.4 against 8.2-9.8 us,
+  // unsteady; 12 rounds of it 9.3 against 10.6); at B <= 4 the halved workgroup
+  // count costs more (12 rounds, B = 1: 8.2 against 7.3), except for f32 activations
   // with Q4_1 and Q8_0 weights (4200 x 3072 Q8_0, B = 4: 7.1 against 7.9).
   if constexpr (NS == 1 && !(CB == 16 && XN) && (CB >= 8 || (CB == 4 && XN && (FMT == GEMV_Q41 || FMT == GEMV_Q8)))) {
     if (p.S > 1 && (int)(grid1.x * grid1.y) > p.ncu) {
@@ -318,7 +316,8 @@ int launch_cb(const GemvParams &p, hipStream_t st) {
     if (p.B <= 2) return launch_one<FMT, NS, EPI, 2, true>(p, st);
     if (p.B <= 4) return launch_one<FMT, NS, EPI, 4, true>(p, st);
     if (p.B <= 8) return launch_one<FMT, NS, EPI, 8, true>(p, st);
-    return launch_one<FMT, NS, EPI, 16, true>(p, st);
+    if constexpr (NS == 1) return launch_one<FMT, NS, EPI, 16, true>(p, st);
+    else return CWEN_EINVAL;   // converted first: see f32_staged
   }
   if (p.B <= 2) return launch_one<FMT, NS, EPI, 2, false>(p, st);
   if (p.B <= 4) return launch_one<FMT, NS, EPI, 4, false>(p, st);
@@ -328,11 +327,10 @@ int launch_cb(const GemvParams &p, hipStream_t st) {
 
 }  // namespace
 
-// The instances whose workgroups may hold more than 64 KB of LDS.
+// The instance whose workgroups may hold more than 64 KB of LDS.
 int gemv_kw_init() {
-  for (const void *k : {(const void *)gemv_kw_kernel<GEMV_Q4, 2, GEMV_EPI_SWIGLU, 16, false, 1>,
-                        (const void *)gemv_kw_kernel<GEMV_Q4, 2, GEMV_EPI_SWIGLU, 16, true, 1>})
-    CWEN_HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kw_lds(2 * KW_MAX, 16, 1)));
+  CWEN_HIP_TRY(hipFuncSetAttribute((const void *)gemv_kw_kernel<GEMV_Q4, 2, GEMV_EPI_SWIGLU, 16, false, 1>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kw_lds(2 * KW_MAX, 16, 1)));
   return CWEN_OK;
 }
 

@@ -384,8 +384,8 @@ def test_elementwise_error_bound(env, kind, K):
 # shorter; more row groups than CUs (two row groups per wave at B > 4, the last
 # one alone, activations staged or converted first); sizes just past each limit
 # (15 rounds at more row groups than CUs, 6 rounds a wave).
-KW_SHAPES = [(16, 32), (17, 480), (100, 2080), (1000, 3072), (4096, 8704), (4100, 2592), (8192, 544), (4300, 7680),
-             (64, 17408)]
+KW_SHAPES = [(16, 32), (17, 480), (100, 2080), (1000, 3072), (4096, 8704), (4100, 2592), (8192, 544), (4300, 7680), (4112, 5120),
+             (64, 17408)]   # (4112, 5120): inside and across workgroups by block size
 
 
 @pytest.mark.parametrize("M,K", KW_SHAPES)
@@ -416,7 +416,7 @@ def test_split_in_workgroup(env, oracle, M, K):
         assert np.array_equal(Y.cpu().numpy(), (Y0[:B].cpu().numpy() + full[:B])), B
 
 
-@pytest.mark.parametrize("M,K", [(40, 96), (1024, 5120), (4096, 1024), (4112, 1024)])
+@pytest.mark.parametrize("M,K", [(40, 96), (1024, 5120), (4096, 1024), (4112, 1024), (1040, 4096)])
 def test_split_in_workgroup_pairs(env, oracle, M, K):
     """Pair, single sides and SwiGLU of small pairs, every block size class."""
     torch, gpu, ctx = env
