@@ -307,9 +307,10 @@ size_t wide_partial_floats(const cwen_weight *w, int nsides, bool finish, int N)
 // The per-position scale of a normalised operand (GemvPost) for N positions;
 // psc holds N floats rounded up to a multiple of 64.
 int wide_scale(const float *ssq, int npart, int K, float eps, int N, float *psc, hipStream_t st);
-// epi STORE or SWIGLU; xh in wide_at's order; psc nullable.
+// epi STORE or SWIGLU; xh in wide_at's order; psc nullable; part: part_floats
+// floats, at least wide_partial_floats.
 int wide_gemm(const cwen_ctx *ctx, const cwen_weight *w, int epi, const _Float16 *xh, int N, const float *psc,
-              const WideOut &o, float *part, hipStream_t st);
+              const WideOut &o, float *part, size_t part_floats, hipStream_t st);
 
 // ------------------------------------------------------------ gdn.hip
 int gdn_block_launch(const cwen_gdn *g, const float *qkv, int qs, const float *z, int zs,

@@ -84,7 +84,7 @@ struct cwen_model {
   float *wX = nullptr, *wssq = nullptr, *wpsc = nullptr;
   float *wlin = nullptr, *wxc = nullptr, *wgates = nullptr;  // in-projection rows; GDN conv values and gates
   float *wq = nullptr, *wpart = nullptr, *watt = nullptr;    // watt: the attention's scores and sums
-  size_t watt_floats = 0;
+  size_t watt_floats = 0, wpart_floats = 0;
   _Float16 *wxh = nullptr, *wgh = nullptr, *whh = nullptr;   // gh: GDN or attention output
   // MTP nextn drafter (blk.N after the N decoder layers; its decoder block
   // is L[n_layers]).  Its KV stream starts at slot 1: slot s lives at index
@@ -462,14 +462,28 @@ void wide_free(cwen_model *m) {
   if (m->hwtok) (void)hipHostFree(m->hwtok);
   m->wtoks = m->hwtok = nullptr;
   m->wX = m->wssq = m->wpsc = m->wlin = m->wxc = m->wgates = m->wq = m->wpart = m->watt = nullptr;
-  m->watt_floats = 0;
+  m->watt_floats = m->wpart_floats = 0;
   m->wxh = m->wgh = m->whh = nullptr;
   m->wn = 0;
 }
 
+// Floats of split-K partials that a pass over N positions of the layers' present
+// weights needs: how a matrix is split depends on its format, and a weight may be
+// replaced by one of another format.
+size_t wide_part_floats(const cwen_model *m, int N) {
+  size_t part = 0;
+  for (int l = 0; l < m->cfg.n_layers; ++l) {
+    const Layer &y = m->L[l];
+    part = std::max({part, wide_partial_floats(y.ffn_gu, 2, false, N), wide_partial_floats(y.ffn_down, 1, true, N),
+                     wide_partial_floats(y.linear ? y.lin_in : y.att_in, 1, false, N),
+                     wide_partial_floats(y.linear ? y.ssm_out : y.wo, 1, true, N)});
+  }
+  return part;
+}
+
 // Workspace for the passes over n positions: their length grows to at most
 // WIDE_MAX, the attention's part with the context (bounded, see
-// attention_wide_floats).
+// attention_wide_floats), the partials with the weights set.
 int wide_alloc(cwen_model *m, int n) {
   const cwen_model_cfg &c = m->cfg;
   int N = std::min(n, WIDE_MAX);
@@ -478,19 +492,13 @@ int wide_alloc(cwen_model *m, int n) {
     const int k = std::min(n - i, WIDE_MAX);
     att = std::max(att, attention_wide_floats(c.n_head, c.n_kv_head, m->pos + 1 + i + k, k));
   }
-  if (m->wn >= N && m->watt_floats >= att) return CWEN_OK;
+  if (m->wn >= N && m->watt_floats >= att && m->wpart_floats >= wide_part_floats(m, N)) return CWEN_OK;
   N = std::max(N, m->wn);
   att = std::max(att, m->watt_floats);
+  const size_t part = wide_part_floats(m, N);
   wide_free(m);
   const Rows R = rows_of(c);
   const size_t np = (size_t)N, H = c.d_model, Qo = (size_t)R.Qo2 / 2;
-  size_t part = 0;
-  for (int l = 0; l < c.n_layers; ++l) {
-    const Layer &y = m->L[l];
-    part = std::max({part, wide_partial_floats(y.ffn_gu, 2, false, N), wide_partial_floats(y.ffn_down, 1, true, N),
-                     wide_partial_floats(y.linear ? y.lin_in : y.att_in, 1, false, N),
-                     wide_partial_floats(y.linear ? y.ssm_out : y.wo, 1, true, N)});
-  }
   // The products read whole tiles of 64 positions, past the last one's end.
   constexpr size_t kSlack = 64 * 128;
   int rc = (dmalloc(&m->wtoks, np) || dmalloc(&m->wX, np * H) || dmalloc(&m->wssq, np * CWEN_MAX_PARTS) ||
@@ -508,6 +516,7 @@ int wide_alloc(cwen_model *m, int n) {
   } else {
     m->wn = N;
     m->watt_floats = att;
+    m->wpart_floats = part;
   }
   return rc;
 }
@@ -534,7 +543,8 @@ int wide_block(cwen_model *m, int N, hipStream_t st) {
     Layer &y = m->L[l];
     if ((rc = wide_scale(m->wssq, npart, H, c.rms_eps, N, m->wpsc, st))) return rc;
     const WideOut oin = {m->wlin, ls, 0, nullptr, nullptr, nullptr, nullptr};
-    if ((rc = wide_gemm(ctx, y.linear ? y.lin_in : y.att_in, GEMV_EPI_STORE, m->wxh, N, m->wpsc, oin, m->wpart, st)))
+    if ((rc = wide_gemm(ctx, y.linear ? y.lin_in : y.att_in, GEMV_EPI_STORE, m->wxh, N, m->wpsc, oin, m->wpart,
+                        m->wpart_floats, st)))
       return rc;
     if (y.linear)
       rc = gdn_wide_launch(y.gdn, m->wlin, ls, r.C, r.o_alpha, r.o_beta, y.ssm_conv, y.ssm_norm, y.ssm_a, y.ssm_dt,
@@ -546,13 +556,13 @@ int wide_block(cwen_model *m, int N, hipStream_t st) {
     if (rc) return rc;
     const cwen_weight *wout = y.linear ? y.ssm_out : y.wo;
     const WideOut oo = {m->wX, H, 1, m->wxh, y.post_norm, m->wssq, rflag};
-    if ((rc = wide_gemm(ctx, wout, GEMV_EPI_STORE, m->wgh, N, nullptr, oo, m->wpart, st)) ||
+    if ((rc = wide_gemm(ctx, wout, GEMV_EPI_STORE, m->wgh, N, nullptr, oo, m->wpart, m->wpart_floats, st)) ||
         (rc = wide_scale(m->wssq, gemv_ssq_parts(wout), H, c.rms_eps, N, m->wpsc, st)))
       return rc;
     const WideOut of = {nullptr, 0, 0, m->whh, nullptr, nullptr, rflag};
     const WideOut od = {m->wX, H, 1, m->wxh, l + 1 < c.n_layers ? m->L[l + 1].attn_norm : m->out_norm, m->wssq, rflag};
-    if ((rc = wide_gemm(ctx, y.ffn_gu, GEMV_EPI_SWIGLU, m->wxh, N, m->wpsc, of, m->wpart, st)) ||
-        (rc = wide_gemm(ctx, y.ffn_down, GEMV_EPI_STORE, m->whh, N, nullptr, od, m->wpart, st)))
+    if ((rc = wide_gemm(ctx, y.ffn_gu, GEMV_EPI_SWIGLU, m->wxh, N, m->wpsc, of, m->wpart, m->wpart_floats, st)) ||
+        (rc = wide_gemm(ctx, y.ffn_down, GEMV_EPI_STORE, m->whh, N, nullptr, od, m->wpart, m->wpart_floats, st)))
       return rc;
     npart = gemv_ssq_parts(y.ffn_down);
   }

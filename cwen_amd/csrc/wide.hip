@@ -366,11 +366,11 @@ int wide_scale(const float *ssq, int npart, int K, float eps, int N, float *psc,
 }
 
 int wide_gemm(const cwen_ctx *ctx, const cwen_weight *w, int epi, const _Float16 *xh, int N, const float *psc,
-              const WideOut &o, float *part, hipStream_t st) {
+              const WideOut &o, float *part, size_t part_floats, hipStream_t st) {
   const int ns = epi == GEMV_EPI_SWIGLU ? 2 : 1;
   const GemvGrid &g = w->cfg[ns - 1];
   const bool finish = epi == GEMV_EPI_STORE && (o.accumulate || o.yh || o.ssq);
-  if (N < 1 || !wide_takes(w, ns, finish)) return CWEN_EINVAL;
+  if (N < 1 || !wide_takes(w, ns, finish) || wide_partial_floats(w, ns, finish, N) > part_floats) return CWEN_EINVAL;
   WideParams p;
   p.w = w->dev;
   p.wbytes = (uint32_t)w->bytes;

@@ -108,6 +108,24 @@ def test_prefill_formats(gpu, types):
     m.free()
 
 
+def test_prefill_after_a_weight_is_replaced(gpu):
+    """The workspace of an earlier prompt part does not bound the pieces of K
+    of a weight set later: ffn_down 4096 x 8192 takes 4 pieces as Q8_0 and,
+    small enough for a workgroup per row group, 6 as Q4_0; no other matrix of
+    this model needs as much room."""
+    cfg = dict(SMALL, n_layers=2, d_model=4096, d_ffn=8192, vocab=1024, full_interval=2)
+    H, I = cfg["d_model"], cfg["d_ffn"]
+    ctx = gpu.Context(0)
+    m = gpu.Model(ctx, **cfg)
+    m.synth(3)
+    for ty, data in ((gpu.T_Q8_0, synth.q8_0(6, H, I)), (gpu.T_Q4_0, synth.q4_gguf(6, H, I)), (gpu.T_Q8_0, synth.q8_0(7, H, I))):
+        print(f"prefill with ffn_down of type {ty}", flush=True)
+        for l in range(cfg["n_layers"]):
+            m.set(l, gpu.FFN_DOWN, ty, data, None, I, H)
+        _compare(gpu, m, cfg, 48)
+    m.free()
+
+
 def test_prefill_refuses(gpu):
     ctx = gpu.Context(0)
     m = gpu.Model(ctx, **SMALL)
