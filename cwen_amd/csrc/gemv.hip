@@ -1062,15 +1062,6 @@ void gemv_choose_split(const cwen_ctx *ctx, cwen_weight *w) {
   w->cfg[2] = w->cfg[0].kw ? w->cfg[0] : grid(2, false);   // inside workgroups the sides are launched side by side
 }
 
-// A weight split inside workgroups whose launch takes the same pieces across
-// workgroups instead (the same sums in the same order): with more row groups than
-// CUs a CU's two workgroups stage the same activations, and from 9 rounds on that
-// shows for f32 ones at B = 3-4.  Inside / across, us: 5120 x 5120 at B = 4 8.5 /
-// 8.25, B = 3 8.2 / 8.2, B = 1 7.5 / 8.2; 6144 x 4096 (8 rounds) at B = 4 7.1 / 8.2.
-static bool kw_across(const cwen_ctx *ctx, const cwen_weight *w, bool f32, int B) {
-  return w->nrg > ctx->ncu && w->nst > 8 && f32 && (B == 3 || B == 4);
-}
-
 int gemv_ssq_parts(const cwen_weight *w) { return w->nrg; }
 
 int gemv_launch(cwen_ctx *ctx, const cwen_weight *w, int nsides, int side0, int epi,
@@ -1106,10 +1097,6 @@ int gemv_launch(cwen_ctx *ctx, const cwen_weight *w, int nsides, int side0, int 
   const int rpw = tile_rows(nsides);
   const int ntile = (w->nrg + rpw - 1) / rpw;
   if (epi == GEMV_EPI_ARGMAX) cfg = {ntile, 0, 1, w->nst, 0, 0};  // final row values in one workgroup
-  if (cfg.kw && cfg.S > 1 && nsides == 1 && kw_across(ctx, w, xf != nullptr, B)) {
-    const GemvGrid a = {ntile * cfg.S, ntile * cfg.S, cfg.S, cfg.rps, 0, 0};
-    if (gemv_grid_fits(a, scr ? scr->partials_floats : ctx->partials_floats, scr ? scr->ncounters : ctx->ncounters)) cfg = a;
-  }
   if (scr && !gemv_grid_fits(cfg, scr->partials_floats, scr->ncounters)) return CWEN_ESCRATCH;
   p.nsplit = cfg.nsplit;
   p.S = cfg.S;

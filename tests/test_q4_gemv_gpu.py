@@ -385,7 +385,7 @@ def test_elementwise_error_bound(env, kind, K):
 # one alone, activations staged or converted first); sizes just past each limit
 # (15 rounds at more row groups than CUs, 6 rounds a wave).
 KW_SHAPES = [(16, 32), (17, 480), (100, 2080), (1000, 3072), (4096, 8704), (4100, 2592), (8192, 544), (4300, 7680), (4112, 5120),
-             (64, 17408)]   # (4112, 5120): inside and across workgroups by block size
+             (64, 17408)]
 
 
 @pytest.mark.parametrize("M,K", KW_SHAPES)
