@@ -971,22 +971,38 @@ double grid_cost(int ncu, int nst, const GemvGrid &c, double extra) {
   return worst + extra;
 }
 
+// The most rounds of K at which a weight of nrg row groups takes the form of
+// gemv_kw.hip (0: never), K split over the waves of one workgroup per row group.
+// It is for at most 18 MB, at most half as many tiles as CUs, and where it was no slower
+// than the forms below: up to 70 % faster at 4 rounds, less as the rounds grow, since each
+// wave stages its own activations for its share of K, however few CUs there are rows
+// for.  Both forms in us, this one first, f16 in, B = 1 / 4 / 8 / 16, weights from HBM, calls
+// replayed from a graph:
+//   Q4_0 6400 x 4096 (400 groups, 8 rounds)    6.1 / 6.5 / 7.0 / 7.5   7.9 / 8.1 / 8.3 / 8.9
+//   Q4_0 2048 x 6144 (128 groups, 12 rounds)   5.3 / 5.7 / 6.0 / 6.8   7.1 / 7.3 / 7.3 / 7.8
+// Fewer row groups than a quarter of the CUs: 13 rounds, 11 with more bytes a round
+// than Q4_1:
+//   Q4_0 512 x 8192 (32 groups, 16 rounds)     6.2 / 6.6 / 7.0 / 8.0   6.3 / 6.4 / 6.5 / 6.9
+// Up to the number of CUs: 14 rounds, Q4_0 15, or 17 from three quarters of the CUs on:
+//   Q8_0 2048 x 7680 (128 groups, 15 rounds)   7.5 / 7.9 / 8.2 / 9.4   7.7 / 7.8 / 7.9 / 8.5
+//   Q4_0 3200 x 8704 (200 groups, 17 rounds)   7.2 / 7.5 / 7.9 / 9.2   8.5 / 8.7 / 8.8 / 9.4
+// More, where some CUs run two workgroups: 8 rounds and 14 MB, Q4_1 9, Q4_0 10:
+//   Q4_0 5120 x 5120 (320 groups, 10 rounds)   7.1 / 7.5 / 8.5 / 9.2   8.1 / 8.2 / 8.4 / 9.0
+//   Q4_1 4224 x 5120 (264 groups, 10 rounds)   7.0 / 7.6 / 8.6 / 9.3   8.1 / 8.2 / 8.2 / 8.7
+//   Q5_K 4224 x 4608 (264 groups, 9 rounds), f32 at B = 4: 10.1 and 8.3
+// What still loses inside these lines: Q4_0 at 10 rounds of more row groups than CUs 1-3 % for
+// B > 4, and Q5_K and Q6_K at 10 rounds of few row groups up to 6 % at B = 16.
+int kw_max_rounds(const cwen_ctx *ctx, int nrg, size_t bytes, int fmt) {
+  const bool q4 = fmt == GEMV_Q4, q41 = fmt == GEMV_Q41;
+  if (bytes > (size_t)18 << 20) return 0;
+  if (nrg > ctx->ncu) return q4 ? 10 : bytes > (size_t)14 << 20 ? 0 : q41 ? 9 : 8;
+  if (4 * nrg < ctx->ncu) return q4 || q41 ? 13 : 11;
+  return !q4 ? 14 : 4 * nrg < 3 * ctx->ncu ? 15 : 17;
+}
+
 // Decomposition of ntile row tiles (nrg row groups) of nst rounds.
-// Small weights (kw): K split over the waves of a workgroup per row group, for
-// about 7 waves per CU, when tiles are at most half as many as CUs, a wave gets
-// at most 3 rounds and the weight has at most 18 MB.  With more row groups than
-// CUs, some of which then run two workgroups, at most 2 rounds of at most 10 and,
-// unless Q4_0, 14 MB: 5120 x 6144 (12 rounds, f32, B = 1 / 4 / 16) 8.7 / 10.0 / 11.5 against
-// 8.4 / 8.5 / 11.2 us, 4300 x 7680 (269 groups, 3 rounds) 8.9-11.9 against 9.0-10.3, Q4_1 5120 x 5120
-// f32 at B = 4 9.1 against 8.2 us.  Measured against the forms below, f16 in, B = 1 / 4 /
-// 8 / 16: 5120 x 5120 7.1 / 7.6 / 8.5 / 9.1 against 8.3 / 8.5 / 8.6 / 9.1 us, 8000 x 2048
-// 4.6 / 4.8 / 4.8 / 5.3 against 6.9 / 7.2 / 7.3 / 8.0, 2048 x 6144 5.1 / 5.8 / 6.1 / 6.9 against
-// 7.4 / 7.6 / 7.7 / 8.0,
-// 1000 x 2080 4.5 / 4.5 / 4.6 / 4.8 against 6.6 / 7.1 / 7.1 / 7.5.  Past it a wave's own
-// activation staging shows: 5120 x 17408 (6 rounds) 15.6 / 17.2 / 19.7 / 26.6
-// against 13.8 / 14.1 / 14.7 / 15.6, Q5_K 5120 x 6144 (23.6 MB) 9.2 / 9.9 / 10.5 /
-// 11.1 against 9.3 / 9.5 / 9.7 / 10.2, 64 x 17408, 4 workgroups, 8.6 against 7.6, and with
-// more tiles 10240 x 2048 at B = 16 8.5 against 6.6.
+// Small weights (kw_max_rounds): K split over the waves of a workgroup, for about
+// 7 waves per CU, at most 3 rounds a wave, or 2 with more row groups than CUs.
 // Otherwise a launch with fewer tiles than CUs splits every tile into S pieces
 // (at least two rounds each) for at most wg_per_cu workgroups per CU.  A larger one takes whole tiles,
 // except that the ntile mod ncu remainder tiles are split into the pieces
@@ -1005,12 +1021,10 @@ double grid_cost(int ncu, int nst, const GemvGrid &c, double extra) {
 // in whole tiles at B = 16).
 GemvGrid choose_grid(const cwen_ctx *ctx, int ntile, int nst, int split_basis, int nrg, size_t bytes, int fmt, bool kw) {
   GemvGrid best = {ntile, 0, 1, nst, 0, 0};
-  if (kw && 2 * split_basis <= ctx->ncu && bytes <= (size_t)18 << 20) {
+  if (kw && 2 * split_basis <= ctx->ncu && nst <= kw_max_rounds(ctx, nrg, bytes, fmt)) {
     const int S0 = std::min({std::max((7 * ctx->ncu + nrg / 2) / nrg, 1), GEMV_KW_MAX, nst});
     const int rps = (nst + S0 - 1) / S0, S = (nst + rps - 1) / rps;
-    const bool one_wave_of_groups = nrg <= ctx->ncu;
-    if (one_wave_of_groups ? rps <= 3 : rps <= 2 && nst <= 10 && (fmt == GEMV_Q4 || bytes <= (size_t)14 << 20))
-      return {ntile * S, ntile * S, S, rps, 0, 1};
+    if (rps <= (nrg <= ctx->ncu ? 3 : 2)) return {ntile * S, ntile * S, S, rps, 0, 1};
   }
   // More than half as many tiles as CUs: whole tiles, one per CU.  Split in
   // two, most CUs would get two pieces of the same total length plus the
