@@ -296,10 +296,11 @@ int launch_one(const GemvParams &p, hipStream_t st) {
   static_assert(CB * NS <= 16 || (FMT == GEMV_Q4 && NS == 2 && CB == 16), "LDS above 64 KB: see gemv_kw_init");
   // Wide blocks over more row groups than CUs: two row groups per wave, which
   // share its staged activations (5120 x 5120, f16, B = 16: 8.4 against 8.2-9.8 us,
-  // unsteady; 12 rounds of it 9.3 against 10.6); at B <= 4 the halved workgroup
-  // count costs more (12 rounds, B = 1: 8.2 against 7.3), except for f32 activations
-  // with Q4_1 and Q8_0 weights (4200 x 3072 Q8_0, B = 4: 7.1 against 7.9).
-  if constexpr (NS == 1 && !(CB == 16 && XN) && (CB >= 8 || (CB == 4 && XN && (FMT == GEMV_Q41 || FMT == GEMV_Q8)))) {
+  // unsteady); at B <= 4 the halved workgroup count costs more (4224 x 5120, f32, B = 3,
+  // weights from HBM: 8.6 against 8.1), except for f32 activations with weights other than
+  // Q4_0 (4224 x 3072 at B = 4, Q5_K 7.2 against 8.0, Q6_K 7.3 against 8.4; 4200 x 3072 Q8_0 7.1
+  // against 7.9, weights in cache).
+  if constexpr (NS == 1 && !(CB == 16 && XN) && (CB >= 8 || (CB == 4 && XN && FMT != GEMV_Q4))) {
     if (p.S > 1 && (int)(grid1.x * grid1.y) > p.ncu) {
       const dim3 grid2((unsigned)((p.nrg + 1) / 2), grid1.y);
       hipLaunchKernelGGL((gemv_kw_kernel<FMT, NS, EPI, CB, XN, 2>), grid2, block, kw_lds(nwave, CB, 2), st, p);

@@ -417,6 +417,29 @@ def test_split_in_workgroup(env, oracle, M, K):
         assert np.array_equal(Y.cpu().numpy(), (Y0[:B].cpu().numpy() + full[:B])), B
 
 
+@pytest.mark.parametrize("kind", ["q8_0", "q6_k", "q4_1", "q5_k"])
+@pytest.mark.parametrize("M,K", [(1000, 1536), (4112, 1024), (4200, 2304), (4112, 3072)])
+def test_split_in_workgroup_formats(env, oracle, kind, M, K):
+    """The formats other than Q4_0: one row group a wave, and (257 and 263 row
+    groups, the last one alone) two; f32 and f16 activations of every block size class."""
+    torch, gpu, ctx = env
+    print(f"split in workgroup {kind} {M}x{K}", flush=True)
+    wtype = {"q8_0": gpu.T_Q8_0, "q4_1": gpu.T_Q4_1, "q6_k": gpu.T_Q6_K, "q5_k": gpu.T_Q5_K}[kind]
+    data = {"q8_0": synth.q8_0, "q4_1": synth.q4_1, "q6_k": synth.q6_k, "q5_k": synth.q5_k}[kind](133, M, K)
+    W = gpu.Weight(ctx, wtype, data, None, K, M)
+    X = synth.activations(133, 16, K)
+    want = oracle.gemvb(wtype, data, None, K, M, X)
+    full = _run(env, W, X)
+    assert rel_err(full, want) <= TOL
+    Xh = torch.from_numpy(X).cuda().half()
+    for B in (1, 3, 4, 5, 8, 9, 16):
+        assert np.array_equal(_run(env, W, X[:B]).view(np.uint32), full[:B].view(np.uint32)), B
+        Y = torch.zeros(B, M, device="cuda")
+        gpu.gemvb_f16(ctx, W, Xh, Y, B)
+        torch.cuda.synchronize()
+        assert np.array_equal(Y.cpu().numpy().view(np.uint32), full[:B].view(np.uint32)), B
+
+
 @pytest.mark.parametrize("M,K", [(40, 96), (1024, 5120), (4096, 1024), (4112, 1024), (1040, 4096)])
 def test_split_in_workgroup_pairs(env, oracle, M, K):
     """Pair, single sides and SwiGLU of small pairs, every block size class."""
