@@ -287,14 +287,14 @@ __global__ __launch_bounds__(64 * RW) void gdn_rec_kernel(GdnParams p) {
     const int b = wave + RW * u;
     if (b >= B) break;
     const float2 o = *(const float2 *)&ob[b][2 * lane];
-    const float ss = sum64(o.x * o.x + o.y * o.y);
+    const float ss = sum64(fmaf(o.x, o.x, o.y * o.y));
     const float sc = 1.f / sqrtf(ss / DK + 1e-6f);
     float2 r;
     r.x = wn2.x * o.x * sc * silu_ref(zr[u].x);
     r.y = wn2.y * o.y * sc * silu_ref(zr[u].y);
     if (p.out) *(float2 *)(p.out + (size_t)b * p.os + hv * DK + 2 * lane) = r;
     if (p.outh) {
-      const half2_t h = {(_Float16)r.x, (_Float16)r.y};
+      const half2_t h = {(_Float16)f32_of(r.x), (_Float16)f32_of(r.y)};
       *(half2_t *)(p.outh + (size_t)b * p.ohs + hv * DK + 2 * lane) = h;
       if (f16_bad(h[0]) || f16_bad(h[1])) raise_flag(p.rflag);
     }
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(256) void gdn_wide_norm_kernel(GdnWide p) {
   const float2 o = *(const float2 *)(p.lin + (size_t)b * p.ls + hv * DK + 2 * lane);
   const float z0 = p.lin[(size_t)b * p.ls + p.zo + hv * DK + 2 * lane];
   const float z1 = p.lin[(size_t)b * p.ls + p.zo + hv * DK + 2 * lane + 1];
-  const float ss = sum64(o.x * o.x + o.y * o.y);
+  const float ss = sum64(fmaf(o.x, o.x, o.y * o.y));
   const float sc = 1.f / sqrtf(ss / DK + 1e-6f);
   float2 r;
   r.x = wn2.x * o.x * sc * silu_ref(z0);

@@ -549,7 +549,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemv_kernel(GemvParams p) {
       if (c >= p.B) continue;
       if (y0) y0[(size_t)c * o.ys + row] = v[e];
       if (o.yh) {
-        const _Float16 h = (_Float16)(o.nwh ? v[e] * nwr : v[e]);
+        const _Float16 h = (_Float16)f32_of(o.nwh ? v[e] * nwr : v[e]);
         o.yh[(size_t)c * p.M + row] = h;
         bad |= f16_bad(h);
       }
