@@ -298,9 +298,18 @@ static bool f32_staged(const cwen_weight *W, int form, int xs, int B) {
   const bool kw = form >= 0 && W->cfg[form].kw;
   return B <= (!kw ? 4 : form == 1 || W->nrg > W->ctx->ncu ? 8 : CWEN_BMAX);
 }
-static int f32_operand(cwen_ctx *ctx, const cwen_weight *W, int form, const float *X, int xs, int B, hipStream_t st,
-                       GemvF32 *n, const _Float16 **xh) {
-  if (f32_staged(W, form, xs, B)) {
+// Whether an output of B columns (nullable) and the activations may share
+// memory: staged, a workgroup may still be reading what another has replaced.
+static bool f32_in_place(const float *X, int xs, int K, const float *Y, int ys, int M, int B) {
+  const uintptr_t x = (uintptr_t)X, y = (uintptr_t)Y;
+  return Y && x < y + ((uintptr_t)(B - 1) * ys + M) * 4 && y < x + ((uintptr_t)(B - 1) * xs + K) * 4;
+}
+// YA, YB (nullable), ys: the outputs.  Blocks past 4 columns may have one of
+// them in X's place, and are then converted first.
+static int f32_operand(cwen_ctx *ctx, const cwen_weight *W, int form, const float *X, int xs, const float *YA,
+                       const float *YB, int ys, int B, hipStream_t st, GemvF32 *n, const _Float16 **xh) {
+  if (f32_staged(W, form, xs, B) && (B <= 4 || !(f32_in_place(X, xs, W->ne0, YA, ys, W->ne1, B) ||
+                                                 f32_in_place(X, xs, W->ne0, YB, ys, W->ne1, B)))) {
     *n = {X, xs};
     *xh = nullptr;
     return CWEN_OK;
@@ -325,7 +334,7 @@ int cwen_gemvb(cwen_ctx *ctx, const cwen_weight *W, int side, const float *X, in
   hipStream_t st = (hipStream_t)stream;
   GemvF32 x;
   const _Float16 *xh;
-  if ((rc = f32_operand(ctx, W, 0, X, xs, B, st, &x, &xh))) return rc;
+  if ((rc = f32_operand(ctx, W, 0, X, xs, Y, nullptr, ys, B, st, &x, &xh))) return rc;
   GemvOut o = {Y, nullptr, nullptr, ys, 0};
   return gemv_launch(ctx, W, 1, side, GEMV_EPI_STORE, xh, o, B, st, xh ? nullptr : &x);
 }
@@ -341,7 +350,7 @@ int cwen_gemvb_pair(cwen_ctx *ctx, const cwen_weight *W, const float *X, int xs,
   hipStream_t st = (hipStream_t)stream;
   GemvF32 x;
   const _Float16 *xh;
-  if ((rc = f32_operand(ctx, W, 2, X, xs, B, st, &x, &xh))) return rc;
+  if ((rc = f32_operand(ctx, W, 2, X, xs, YA, YB, ys, B, st, &x, &xh))) return rc;
   GemvOut o = {YA, YB, nullptr, ys, 0};
   return gemv_launch(ctx, W, 2, 0, GEMV_EPI_PAIR, xh, o, B, st, xh ? nullptr : &x);
 }
@@ -355,7 +364,7 @@ int cwen_gemvb_swiglu(cwen_ctx *ctx, const cwen_weight *W, const float *X, int x
   hipStream_t st = (hipStream_t)stream;
   GemvF32 x;
   const _Float16 *xh;
-  if ((rc = f32_operand(ctx, W, 1, X, xs, B, st, &x, &xh))) return rc;
+  if ((rc = f32_operand(ctx, W, 1, X, xs, H, nullptr, hs, B, st, &x, &xh))) return rc;
   GemvOut o = {H, nullptr, nullptr, hs, 0};
   return gemv_launch(ctx, W, 2, 0, GEMV_EPI_SWIGLU, xh, o, B, st, xh ? nullptr : &x);
 }
@@ -394,7 +403,7 @@ int cwen_mlp_block(cwen_ctx *ctx, const cwen_weight *Wgu, const cwen_weight *Wd,
   hipStream_t st = (hipStream_t)stream;
   GemvF32 x;
   const _Float16 *xh;
-  if ((rc = f32_operand(ctx, Wgu, 1, X, xs, B, st, &x, &xh))) return rc;
+  if ((rc = f32_operand(ctx, Wgu, 1, X, xs, nullptr, nullptr, 0, B, st, &x, &xh))) return rc;
   GemvOut o1 = {nullptr, nullptr, ctx->hh, 0, 0};
   if ((rc = gemv_launch(ctx, Wgu, 2, 0, GEMV_EPI_SWIGLU, xh, o1, B, st, xh ? nullptr : &x))) return rc;
   GemvOut o2 = {Y, nullptr, nullptr, ys, 1};
@@ -442,7 +451,7 @@ int cwen_head_verify(cwen_ctx *ctx, const cwen_weight *W, const float *X, int xs
   hipStream_t st = (hipStream_t)stream;
   GemvF32 x;
   const _Float16 *xh;
-  if ((rc = f32_operand(ctx, W, -1, X, xs, B, st, &x, &xh))) return rc;
+  if ((rc = f32_operand(ctx, W, -1, X, xs, logits, nullptr, ls, B, st, &x, &xh))) return rc;
   GemvOut o = {logits, nullptr, nullptr, ls, 0, {ctx->amax_keys, ctx->amax_cnt, drafts, E, res}};
   return gemv_launch(ctx, W, 1, 0, GEMV_EPI_ARGMAX, xh, o, B, st, xh ? nullptr : &x);
 }

@@ -100,8 +100,11 @@ int cwen_weight_info(const cwen_weight *w, int *type, int *ne0, int *ne1,
  * Per output the arithmetic does not depend on B or on the other columns,
  * so a column computed in a block is bit-identical to the same column
  * computed alone.  Replaces gemvb (run.c:1577-1680) and, at B=1, gemv
- * (run.c:1419-1527).  X is converted to the f16 operand format in the
- * context's scratch first (a second, small launch on the same stream). */
+ * (run.c:1419-1527).  X is converted to the f16 operand format first: in the
+ * context's scratch (a second, small launch on the same stream) or, for small
+ * blocks and small weights, by the launch itself.  Y may overlap X only for
+ * B > 4; such a block takes the scratch.  This holds for the other entry points
+ * with f32 activations too. */
 int cwen_gemvb(cwen_ctx *ctx, const cwen_weight *W, int side,
                const float *X, int xs, float *Y, int ys, int B, void *stream);
 

@@ -417,6 +417,43 @@ def test_split_in_workgroup(env, oracle, M, K):
         assert np.array_equal(Y.cpu().numpy(), (Y0[:B].cpu().numpy() + full[:B])), B
 
 
+@pytest.mark.parametrize("n", [1024, 4160, 5120])
+def test_output_in_place_of_the_activations(env, n):
+    """Blocks past 4 columns whose output overwrites their f32 activations, where
+    the launch would otherwise stage these itself: single, one output of a pair,
+    SwiGLU, and an output that starts in the last column."""
+    torch, gpu, ctx = env
+    print(f"in place {n}", flush=True)
+    qs, sc = synth.q4_rs(134, n, n)
+    W = gpu.Weight(ctx, T_RS, qs, sc, n, n)
+    pqs, psc = synth.q4_rsi(134, n, n)
+    P = gpu.Weight(ctx, T_RSI, pqs, psc, n, n)
+    X = synth.activations(134, 16, n)
+    for B in (5, 8, 9, 16):
+        buf = torch.zeros(2 * B, n, device="cuda")
+        other = torch.zeros(B, n, device="cuda")
+        x = torch.from_numpy(X[:B]).cuda()
+
+        def fresh(at):
+            buf[at:at + B] = x
+            torch.cuda.synchronize()
+            return buf[at:at + B]
+
+        want = _run(env, W, X[:B])
+        gpu.gemvb(ctx, W, fresh(0), buf, B)
+        assert np.array_equal(buf[:B].cpu().numpy(), want), B
+        gpu.gemvb(ctx, W, fresh(0), buf[B - 1:], B)
+        assert np.array_equal(buf[B - 1:2 * B - 1].cpu().numpy(), want), B
+        wa, wb = _run(env, P, X[:B], mode="pair")
+        gpu.gemvb_pair(ctx, P, fresh(0), buf, other, B)
+        assert np.array_equal(buf[:B].cpu().numpy(), wa) and np.array_equal(other.cpu().numpy(), wb), B
+        gpu.gemvb_pair(ctx, P, fresh(0), other, buf, B)
+        assert np.array_equal(buf[:B].cpu().numpy(), wb) and np.array_equal(other.cpu().numpy(), wa), B
+        want = _run(env, P, X[:B], mode="swiglu")
+        gpu.gemvb_swiglu(ctx, P, fresh(0), buf, B)
+        assert np.array_equal(buf[:B].cpu().numpy(), want), B
+
+
 @pytest.mark.parametrize("kind", ["q8_0", "q6_k", "q4_1", "q5_k"])
 @pytest.mark.parametrize("M,K", [(1000, 1536), (4112, 1024), (4200, 2304), (4112, 3072)])
 def test_split_in_workgroup_formats(env, oracle, kind, M, K):
