@@ -91,20 +91,25 @@ def test_prefill_equals_blocks(gpu, name, n, n2):
     m.free()
 
 
+@pytest.mark.parametrize("streams", [1, 4])
 @pytest.mark.parametrize("types", [("q8_0", "q6_k"), ("q5_k", "q4_1"), ("q4_0", "q8_0")])
-def test_prefill_formats(gpu, types):
-    """ssm_out / wo and ffn_down in each format the layers take."""
-    print(f"prefill formats {types}", flush=True)
+def test_prefill_formats(gpu, types, streams):
+    """ssm_out / wo and ffn_down in each format the layers take, in the products'
+    two forms: one row stream per wave (1024 rows, 176 positions: at most 3 tiles
+    of positions x 16 row blocks x 4 pieces), and four (2048 x 2048 at 528 positions:
+    9 x 8 x 4 pieces, more workgroups than CUs; the last tile has 16 positions)."""
+    print(f"prefill formats {types}, {streams} streams", flush=True)
     ctx = gpu.Context(0)
-    m = gpu.Model(ctx, **SMALL)
+    cfg, n = (SMALL, 176) if streams == 1 else (dict(SMALL, d_model=2048, n_head=8, gdn_nkh=4, gdn_nvh=16), 528)
+    m = gpu.Model(ctx, **cfg)
     tid = {"q8_0": gpu.T_Q8_0, "q6_k": gpu.T_Q6_K, "q5_k": gpu.T_Q5_K, "q4_1": gpu.T_Q4_1, "q4_0": gpu.T_Q4_0}
     gen = {"q8_0": synth.q8_0, "q6_k": synth.q6_k, "q5_k": synth.q5_k, "q4_1": synth.q4_1, "q4_0": synth.q4_gguf}
-    for l, t, ty, data, sc, ne0, ne1 in synth.model_tensors(SMALL, seed=4):
+    for l, t, ty, data, sc, ne0, ne1 in synth.model_tensors(cfg, seed=4):
         if t in (gpu.SSM_OUT, gpu.ATTN_OUTPUT, gpu.FFN_DOWN):
             f = types[t == gpu.FFN_DOWN]
             ty, data, sc = tid[f], gen[f](5, ne1, ne0, key=100 * l + t), None
         m.set(l, t, ty, data, sc, ne0, ne1)
-    _compare(gpu, m, SMALL, 176)
+    _compare(gpu, m, cfg, n)
     m.free()
 
 
