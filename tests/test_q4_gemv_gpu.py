@@ -417,6 +417,35 @@ def test_split_in_workgroup(env, oracle, M, K):
         assert np.array_equal(Y.cpu().numpy(), (Y0[:B].cpu().numpy() + full[:B])), B
 
 
+@pytest.mark.parametrize("kind", ["rs", "q8_0", "q6_k", "q4_1", "q5_k"])
+@pytest.mark.parametrize("M,K", [(100, 8192), (8250, 768)])
+def test_formats_past_the_small_weights(env, oracle, kind, M, K):
+    """Every format in the two other forms: K split across workgroups (16
+    rounds of few rows) and whole row tiles (130 of them), both ragged; f32
+    activations staged and converted first, and f16 ones."""
+    torch, gpu, ctx = env
+    print(f"past the small weights {kind} {M}x{K}", flush=True)
+    if kind == "rs":
+        wtype = T_RS
+        data, sc = synth.q4_rs(135, M, K)
+    else:
+        wtype = {"q8_0": gpu.T_Q8_0, "q4_1": gpu.T_Q4_1, "q6_k": gpu.T_Q6_K, "q5_k": gpu.T_Q5_K}[kind]
+        data = {"q8_0": synth.q8_0, "q4_1": synth.q4_1, "q6_k": synth.q6_k, "q5_k": synth.q5_k}[kind](135, M, K)
+        sc = None
+    W = gpu.Weight(ctx, wtype, data, sc, K, M)
+    X = synth.activations(135, 16, K)
+    want = oracle.gemvb(wtype, data, sc, K, M, X)
+    full = _run(env, W, X)
+    assert rel_err(full, want) <= TOL
+    Xh = torch.from_numpy(X).cuda().half()
+    for B in (1, 4, 5, 8, 16):
+        assert np.array_equal(_run(env, W, X[:B]).view(np.uint32), full[:B].view(np.uint32)), B
+        Y = torch.zeros(B, M, device="cuda")
+        gpu.gemvb_f16(ctx, W, Xh, Y, B)
+        torch.cuda.synchronize()
+        assert np.array_equal(Y.cpu().numpy().view(np.uint32), full[:B].view(np.uint32)), B
+
+
 @pytest.mark.parametrize("n", [1024, 4160, 5120])
 def test_output_in_place_of_the_activations(env, n):
     """Blocks past 4 columns whose output overwrites their f32 activations, where
