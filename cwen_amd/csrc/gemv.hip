@@ -980,10 +980,11 @@ double grid_cost(int ncu, int nst, const GemvGrid &c, double extra) {
 // replayed from a graph:
 //   Q4_0 6400 x 4096 (400 groups, 8 rounds)    6.1 / 6.5 / 7.0 / 7.5   7.9 / 8.1 / 8.3 / 8.9
 //   Q4_0 2048 x 6144 (128 groups, 12 rounds)   5.3 / 5.7 / 6.0 / 6.8   7.1 / 7.3 / 7.3 / 7.8
-// Fewer row groups than a quarter of the CUs: 13 rounds, 11 with more bytes a round
-// than Q4_1:
+// Fewer row groups than an eighth of the CUs: 13 rounds, 11 with more bytes a round than
+// Q4_1.  Up to a quarter: 13, Q4_1 14, Q4_0 15:
+//   Q4_0 512 x 7680 (32 groups, 15 rounds)     6.1 / 6.5 / 6.9 / 7.8   6.7 / 6.9 / 6.9 / 7.4
 //   Q4_0 512 x 8192 (32 groups, 16 rounds)     6.2 / 6.6 / 7.0 / 8.0   6.3 / 6.4 / 6.5 / 6.9
-// Up to the number of CUs: 14 rounds, Q4_0 15, or 17 from three quarters of the CUs on:
+// Up to the number of CUs: 14, Q4_0 15, or 17 from three quarters of the CUs on:
 //   Q8_0 2048 x 7680 (128 groups, 15 rounds)   7.5 / 7.9 / 8.2 / 9.4   7.7 / 7.8 / 7.9 / 8.5
 //   Q4_0 3200 x 8704 (200 groups, 17 rounds)   7.2 / 7.5 / 7.9 / 9.2   8.5 / 8.7 / 8.8 / 9.4
 // More, where some CUs run two workgroups: 8 rounds and 14 MB, Q4_1 9, Q4_0 10:
@@ -991,12 +992,13 @@ double grid_cost(int ncu, int nst, const GemvGrid &c, double extra) {
 //   Q4_1 4224 x 5120 (264 groups, 10 rounds)   7.0 / 7.6 / 8.6 / 9.3   8.1 / 8.2 / 8.2 / 8.7
 //   Q5_K 4224 x 4608 (264 groups, 9 rounds), f32 at B = 4: 10.1 and 8.3
 // What still loses inside these lines: Q4_0 at 10 rounds of more row groups than CUs 1-3 % for
-// B > 4, and Q5_K and Q6_K at 10 rounds of few row groups up to 6 % at B = 16.
+// B > 4; Q5_K and Q6_K at 10 rounds of few row groups, and Q4_0 at 15 of 32, up to 6 % at B = 16.
 int kw_max_rounds(const cwen_ctx *ctx, int nrg, size_t bytes, int fmt) {
   const bool q4 = fmt == GEMV_Q4, q41 = fmt == GEMV_Q41;
   if (bytes > (size_t)18 << 20) return 0;
   if (nrg > ctx->ncu) return q4 ? 10 : bytes > (size_t)14 << 20 ? 0 : q41 ? 9 : 8;
-  if (4 * nrg < ctx->ncu) return q4 || q41 ? 13 : 11;
+  if (8 * nrg < ctx->ncu) return q4 || q41 ? 13 : 11;
+  if (4 * nrg < ctx->ncu) return q4 ? 15 : q41 ? 14 : 13;
   return !q4 ? 14 : 4 * nrg < 3 * ctx->ncu ? 15 : 17;
 }
 

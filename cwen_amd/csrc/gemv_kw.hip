@@ -299,8 +299,8 @@ int launch_one(const GemvParams &p, hipStream_t st) {
   // unsteady); at B <= 4 the halved workgroup count costs more (4224 x 5120, f32, B = 3,
   // weights from HBM: 8.6 against 8.1), except for f32 activations with weights other than
   // Q4_0 (4224 x 3072 at B = 4, Q5_K 7.2 against 8.0, Q6_K 7.3 against 8.4; 4200 x 3072 Q8_0 7.1
-  // against 7.9, weights in cache).
-  if constexpr (NS == 1 && !(CB == 16 && XN) && (CB >= 8 || (CB == 4 && XN && FMT != GEMV_Q4))) {
+  // against 7.9, weights in cache).  A pair's two sides never exceed the CUs here.
+  if constexpr (NS == 1 && EPI != GEMV_EPI_PAIR && !(CB == 16 && XN) && (CB >= 8 || (CB == 4 && XN && FMT != GEMV_Q4))) {
     if (p.S > 1 && (int)(grid1.x * grid1.y) > p.ncu) {
       const dim3 grid2((unsigned)((p.nrg + 1) / 2), grid1.y);
       hipLaunchKernelGGL((gemv_kw_kernel<FMT, NS, EPI, CB, XN, 2>), grid2, block, kw_lds(nwave, CB, 2), st, p);
@@ -314,11 +314,15 @@ int launch_one(const GemvParams &p, hipStream_t st) {
 template <int FMT, int NS, int EPI>
 int launch_cb(const GemvParams &p, hipStream_t st) {
   if (p.xf) {
-    if (p.B <= 2) return launch_one<FMT, NS, EPI, 2, true>(p, st);
-    if (p.B <= 4) return launch_one<FMT, NS, EPI, 4, true>(p, st);
-    if (p.B <= 8) return launch_one<FMT, NS, EPI, 8, true>(p, st);
-    if constexpr (NS == 1) return launch_one<FMT, NS, EPI, 16, true>(p, st);
-    else return CWEN_EINVAL;   // converted first: see f32_staged
+    if constexpr (EPI == GEMV_EPI_CONV) {
+      return CWEN_EINVAL;      // the model's operands are f16
+    } else {
+      if (p.B <= 2) return launch_one<FMT, NS, EPI, 2, true>(p, st);
+      if (p.B <= 4) return launch_one<FMT, NS, EPI, 4, true>(p, st);
+      if (p.B <= 8) return launch_one<FMT, NS, EPI, 8, true>(p, st);
+      if constexpr (NS == 1) return launch_one<FMT, NS, EPI, 16, true>(p, st);
+      else return CWEN_EINVAL;   // converted first: see f32_staged
+    }
   }
   if (p.B <= 2) return launch_one<FMT, NS, EPI, 2, false>(p, st);
   if (p.B <= 4) return launch_one<FMT, NS, EPI, 4, false>(p, st);

@@ -382,10 +382,10 @@ def test_elementwise_error_bound(env, kind, K):
 # Weights small enough for K to be split over a workgroup's waves: one wave and
 # one round; rows and K ragged; the most pieces, of 3 rounds with one of 2 last; more
 # row groups than CUs (two row groups per wave at B > 4, the last one alone, activations
-# staged or converted first).  Then both sides of each limit: 14 rounds at 63 and 64 row
+# staged or converted first).  Then both sides of each limit: 14 rounds at 31 and 32 row
 # groups, 15 and 16 at 64, 10 and 11 at 257, and two far past it.
 KW_SHAPES = [(16, 32), (17, 480), (100, 2080), (1000, 3072), (3200, 8704), (4100, 2592), (8192, 544),
-             (1008, 7008), (1010, 7008), (1024, 7680), (1024, 8192), (4112, 5120), (4112, 5152),
+             (496, 7008), (500, 7008), (1024, 7680), (1024, 8192), (4112, 5120), (4112, 5152),
              (4300, 7680), (64, 17408)]
 
 
