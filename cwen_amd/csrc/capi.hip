@@ -506,10 +506,11 @@ int cwen_gdn_free(cwen_gdn *g) {
   return CWEN_OK;
 }
 
-// Write the host copy of the control word where captured blocks read it (after
-// queued work): mapped host memory, so that this is four stores.  As a 16-byte
-// copy to the device a commit took 20.7 us, with nothing queued before it; so
-// 0.6 us.  Blocks outside a capture get the word by value.
+// Write the host copy of the control word where captured blocks read it: mapped
+// host memory, so that this is four stores.  It waits for the whole device first, since a
+// replay that reads the word may be queued on any stream.  As a 16-byte copy to the
+// device a commit took 20.7 us with nothing queued before it; so 0.6 us.  Blocks
+// outside a capture get the word by value.
 static int gdn_sync_ctl(cwen_gdn *g) {
   CWEN_HIP_TRY(hipDeviceSynchronize());
   const int c[4] = {g->cur, g->X, g->L, g->P};

@@ -8,8 +8,8 @@
 // short-walk replay 4975-4988 are replaced as below.
 //
 // Per position b (C = 2*nkh*dk + nvh*dk channels):
-//   conv:  x_c = st0*w0 + st1*w1 + st2*w2 + cur*w3 (no FMA contraction, the
-//          reference's scalar order), history shifts in cur, x = silu(x)
+//   conv:  x_c = st0*w0 + st1*w1 + st2*w2 + cur*w3 (one product and three
+//          FMAs, conv4), history shifts in cur, x = silu(x)
 //   q, k:  l2-normalised per key head, x / sqrt(sum x^2 + 1e-6)
 //   per value head hv (key head hv % nkh):
 //          S *= exp(decay);  sk = S^T k;  delta = beta (v - sk);
@@ -87,7 +87,7 @@ struct GdnParams {
 // position (blockIdx.y).  The 4-tap filter needs no running state: the
 // inputs at b-3 .. b-1 come from the block's own rows or, before the block,
 // from the history slot the block starts from, so every position is
-// computed at once with run.c's product/sum order.  The pending buffer
+// computed at once (conv4, as every conv path).  The pending buffer
 // holds the post-conv values; the recurrence l2-normalises q and k as it
 // stages them, for the block and for a later replay alike.  Each position's
 // thread also writes that position's history slot (inputs b-2, b-1, b).

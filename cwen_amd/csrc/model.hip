@@ -63,8 +63,9 @@ __device__ __forceinline__ void embed_block_q6k(const uint8_t *row, int i, float
 
 // A thread dequantizes one 32-weight block and adds its squares (the order of
 // the row's sum); the values pass through LDS so that they leave 16 bytes per
-// lane side by side.  Stored straight from the dequantizing thread, 81 stores of 4
-// or 2 bytes a 32-weight block apart, the launch took 12.1 us in a decode step; so 5.7 us.
+// lane side by side.  Stored straight from the dequantizing thread, 32 stores of 4
+// bytes and 32 of 2, each 32 weights from the next thread's, the launch took 12.1 us in
+// a decode step; so 5.7 us.
 __global__ __launch_bounds__(256) void embed_kernel(const uint8_t *qs, const uint16_t *sc, int type,
                                                     const int *toks, int H, float *X, int xs, float *ssq,
                                                     _Float16 *xh, const float *nw, int *rflag, int tiled, EmbedToks tv) {

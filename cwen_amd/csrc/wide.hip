@@ -25,9 +25,12 @@
 // operands: with 8 position tiles and one workgroup per CU the compiler spilled
 // loads in flight (739 us for gate/up below), and 8 position tiles of 2 streams,
 // half the unpacking per product, came to the same time as this (395 us).
-// Measured, gate/up 2 x 17408 x 5120 at 1024 positions: 392 us, 0.93 PFLOP/s
+// Measured, gate/up 2 x 17408 x 5120 at 1024 positions: 392-408 us, 0.90-0.93 PFLOP/s
 // (a library f16 product of 8192^3 on the same card: 1.18).  4096 positions at
-// 4 layers of the 27B shape: 97.6 ms in blocks of 16, 28.1 ms in passes of 1024.
+// 4 layers of the 27B shape: 97 ms in blocks of 16, 20.6 ms in passes of 1024.
+// The registers fit Q4_0 (2 spilled).  With SPW = 4 the other formats spill: Q4_1 42, Q8_0 59,
+// Q5_K 99, Q6_K 115 registers a lane.  The same prompt with Q5_K out- and Q4_1
+// down-projections takes 24.6 ms (98.5 in blocks), with Q8_0 and Q6_K 29.7 (102).
 #include <algorithm>
 
 #include "cwen_internal.h"
@@ -37,7 +40,6 @@ namespace {
 
 constexpr int WW = 4;                // waves per workgroup
 constexpr int TG = 4;                // row groups of a single-sided row tile of gemv_kernel
-
 
 struct WideParams {
   const uint8_t *w;
@@ -207,7 +209,7 @@ __global__ __launch_bounds__(64 * WW, P * SPW > 16 ? 1 : 2) void wide_kernel(Wid
 
   // One 128-K tile per step.  The scheduling barriers keep the request order
   // (activations of tile t + 2, weights of tile t + 1) and one K run's operands
-  // live at a time: without them the scheduler hoists reads until it spills.
+  // live at a time: without them the scheduler hoists reads until Q4_0 spills too.
   for (int r = 0; r < nround; ++r) {
 #pragma unroll
     for (int u = 0; u < Q4_ST_TILES; ++u) {
