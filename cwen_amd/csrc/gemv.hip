@@ -974,19 +974,19 @@ double grid_cost(int ncu, int nst, const GemvGrid &c, double extra) {
 // The most rounds of K at which a weight of nrg row groups takes the form of
 // gemv_kw.hip (0: never), K split over the waves of one workgroup per row group.
 // It is for at most 18 MB, at most half as many tiles as CUs, and where it was no slower
-// than the forms below: up to 70 % faster at 4 rounds, less as the rounds grow, since each
-// wave stages its own activations for its share of K, however few CUs there are rows
-// for.  Both forms in us, this one first, f16 in, B = 1 / 4 / 8 / 16, weights from HBM, calls
-// replayed from a graph:
+// than the forms below: up to 70 % faster at 4 rounds, less as the rounds grow, since
+// each wave stages the activations of its share of K for itself.  Both forms in us, this one
+// first, f16 in, B = 1 / 4 / 8 / 16, weights from HBM, calls replayed from a graph:
 //   Q4_0 6400 x 4096 (400 groups, 8 rounds)    6.1 / 6.5 / 7.0 / 7.5   7.9 / 8.1 / 8.3 / 8.9
 //   Q4_0 2048 x 6144 (128 groups, 12 rounds)   5.3 / 5.7 / 6.0 / 6.8   7.1 / 7.3 / 7.3 / 7.8
 // Fewer row groups than an eighth of the CUs: 13 rounds, 11 with more bytes a round than
 // Q4_1.  Up to a quarter: 13, Q4_1 14, Q4_0 15:
 //   Q4_0 512 x 7680 (32 groups, 15 rounds)     6.1 / 6.5 / 6.9 / 7.8   6.7 / 6.9 / 6.9 / 7.4
 //   Q4_0 512 x 8192 (32 groups, 16 rounds)     6.2 / 6.6 / 7.0 / 8.0   6.3 / 6.4 / 6.5 / 6.9
-// Up to the number of CUs: 14, Q4_0 15, or 17 from three quarters of the CUs on:
+// Up to the number of CUs: 14, Q4_0 15; from three quarters of them on Q4_0 and Q4_1 17:
 //   Q8_0 2048 x 7680 (128 groups, 15 rounds)   7.5 / 7.9 / 8.2 / 9.4   7.7 / 7.8 / 7.9 / 8.5
 //   Q4_0 3200 x 8704 (200 groups, 17 rounds)   7.2 / 7.5 / 7.9 / 9.2   8.5 / 8.7 / 8.8 / 9.4
+//   Q4_1 3072 x 8704 (192 groups, 17 rounds)   7.3 / 7.8 / 8.3 / 9.2   8.4 / 8.6 / 8.8 / 9.3
 // More, where some CUs run two workgroups: 8 rounds and 14 MB, Q4_1 9, Q4_0 10:
 //   Q4_0 5120 x 5120 (320 groups, 10 rounds)   7.1 / 7.5 / 8.5 / 9.2   8.1 / 8.2 / 8.4 / 9.0
 //   Q4_1 4224 x 5120 (264 groups, 10 rounds)   7.0 / 7.6 / 8.6 / 9.3   8.1 / 8.2 / 8.2 / 8.7
@@ -999,7 +999,7 @@ int kw_max_rounds(const cwen_ctx *ctx, int nrg, size_t bytes, int fmt) {
   if (nrg > ctx->ncu) return q4 ? 10 : bytes > (size_t)14 << 20 ? 0 : q41 ? 9 : 8;
   if (8 * nrg < ctx->ncu) return q4 || q41 ? 13 : 11;
   if (4 * nrg < ctx->ncu) return q4 ? 15 : q41 ? 14 : 13;
-  return !q4 ? 14 : 4 * nrg < 3 * ctx->ncu ? 15 : 17;
+  return (q4 || q41) && 4 * nrg >= 3 * ctx->ncu ? 17 : q4 ? 15 : 14;
 }
 
 // Decomposition of ntile row tiles (nrg row groups) of nst rounds.

@@ -383,8 +383,8 @@ def test_elementwise_error_bound(env, kind, K):
 # one round; rows and K ragged; the most pieces, of 3 rounds with one of 2 last; more
 # row groups than CUs (two row groups per wave at B > 4, the last one alone, activations
 # staged or converted first).  Then both sides of each limit: 14 rounds at 31 and 32 row
-# groups, 15 and 16 at 64, 10 and 11 at 257, and two far past it.
-KW_SHAPES = [(16, 32), (17, 480), (100, 2080), (1000, 3072), (3200, 8704), (4100, 2592), (8192, 544),
+# groups, 15 and 16 at 64, 17 at 191 and 200, 10 and 11 at 257, and two far past it.
+KW_SHAPES = [(16, 32), (17, 480), (100, 2080), (1000, 3072), (3200, 8704), (3056, 8704), (4100, 2592), (8192, 544),
              (496, 7008), (500, 7008), (1024, 7680), (1024, 8192), (4112, 5120), (4112, 5152),
              (4300, 7680), (64, 17408)]
 
